@@ -133,6 +133,10 @@ int pct_ctx_create(const pct_params* p, int device, pct_ctx** out)
         if (t >= 1 && t <= 512) ctx->carve_spill = t;
     }
     if (const char* e = std::getenv("PCT_DROP_PIPELINE")) ctx->drop_pipeline = std::atoi(e) != 0;
+    if (const char* e = std::getenv("PCT_DROP_TILES")) {
+        int t = std::atoi(e);
+        if (t >= -1 && t <= 1) ctx->drop_tiles = t;
+    }
     if (const char* e = std::getenv("PCT_MLP_BLOCKS_PER_CU")) {
         int b = std::atoi(e);
         if (b >= -1 && b <= 64) ctx->mlp_blocks_per_cu = b;
@@ -589,8 +593,9 @@ const char* pct_metrics_json(pct_ctx* ctx)
     }
     std::snprintf(buf, sizeof(buf), "}, \"kernel_ms\": {\"mlp_lists\": %.4f}", ctx->t_mlp_kernel);
     s += buf;
-    std::snprintf(buf, sizeof(buf), ", \"drop_plan\": {\"flags\": %d, \"groups_bucketed\": %lld, \"groups_sorted\": %lld}",
-                  ctx->plan.flags, (long long)ctx->plan.groups_bucketed, (long long)ctx->plan.groups_sorted);
+    std::snprintf(buf, sizeof(buf), ", \"drop_plan\": {\"flags\": %d, \"groups_bucketed\": %lld, \"groups_sorted\": %lld, \"tiles\": %s}",
+                  ctx->plan.flags, (long long)ctx->plan.groups_bucketed, (long long)ctx->plan.groups_sorted,
+                  ctx->plan.tile.ready ? "true" : "false");
     s += buf;
     double tvs_ms = 0;
     for (const TvsRecord& r : ctx->tvs_log) tvs_ms += r.ms;

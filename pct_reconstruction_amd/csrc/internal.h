@@ -76,6 +76,69 @@ struct SliceBlock {
     uint32_t n_vox, pad;
 };
 
+// DROP over image tiles (k_drop_tiles.hip).
+struct TileRow {   // per reconstruction history, in visiting order
+    int64_t off;   // first list entry
+    double chord;  // effective chord length
+    uint32_t cnt;  // list length
+    float wepl;
+    uint32_t seg, n_seg;  // its segments: place[seg .. seg + n_seg) of the group
+};
+struct TileRun {  // one (block, tile) of a group
+    uint32_t key, seg, n;  // first segment, segments | touched voxels << 16
+    uint32_t entries, col, row, pad;  // list entries, and where its lists start (64-word units)
+    uint64_t cw, rw[2];    // units of every slice of voxels and of segments, one byte each
+};
+struct alignas(64) TileDesc {  // one (block, used tile)
+    uint32_t seg, n, run, col, row, tile;
+    uint64_t cw, rw[2], spare[2];
+};
+struct RowPart {  // partial row sum of one segment and the bounds of its tile's values
+    double sum;
+    int32_t top, lsb;
+};
+struct BlockTotals {  // per raw block: touched voxels, list entries, first segment in its group
+    uint32_t touched, entries, seg;
+};
+struct TileGroup {
+    uint32_t segs = 0, n_runs = 0;
+    uint32_t *seg_rank = nullptr, *seg_ord = nullptr, *place = nullptr;
+    uint16_t* tv = nullptr;
+    TileRun* runs = nullptr;
+    uint32_t* words = nullptr;    // column and row lists
+    int64_t entries_hint = 0;     // list slots of the group
+    int64_t cap_seg_rank = 0, cap_seg_ord = 0, cap_place = 0, cap_tv = 0, cap_runs = 0, cap_words = 0;
+};
+struct TileScratch {  // of a group's build
+    uint32_t *hkey = nullptr, *hidx = nullptr, *nseg = nullptr, *q0 = nullptr, *keys = nullptr;
+    uint32_t *idx = nullptr, *runs = nullptr, *n_runs = nullptr, *limits = nullptr, *need = nullptr;
+    uint4* recs = nullptr;  // segment records, then the sorted ones
+    uint64_t* cursor = nullptr;
+    int64_t cap_hkey = 0, cap_hidx = 0, cap_nseg = 0, cap_q0 = 0, cap_keys = 0, cap_idx = 0,
+            cap_runs = 0, cap_recs = 0, cap_need = 0;
+};
+struct TilePlan {
+    std::vector<TileGroup> groups;
+    TileScratch scratch;
+    TileRow* rows = nullptr;
+    uint8_t* used = nullptr;       // per tile: touched by some block
+    uint32_t* index_of = nullptr;  // per tile: its place among the used ones
+    int32_t* block_of = nullptr;   // per raw block: its plan block
+    BlockTotals* totals = nullptr; // per raw block
+    TileDesc* table = nullptr;     // [block][used tile]
+    RowPart* part = nullptr;       // per segment of the next block
+    double* r = nullptr;           // per rank of the current block: the update value of that history
+    float* x = nullptr;            // the image in tiles
+    std::vector<uint32_t> block_seg;  // per block: its first segment in its group
+    int64_t n_used = 0, max_seg = 0;
+    double too_dense = 1e30;       // slots per block and tile at which a list build found a tile too full
+    int64_t cap_rows = 0, cap_used = 0, cap_index_of = 0, cap_block_of = 0, cap_totals = 0,
+            cap_table = 0, cap_part = 0, cap_r = 0, cap_x = 0;
+    bool ready = false;
+};
+constexpr int64_t kTileGroupEntries = 1ll << 30;  // list slots per group of blocks
+constexpr int64_t kMaxTable = 1ll << 26;          // (block, used tile) descriptors
+
 struct DropPlan {
     struct Block {
         int64_t start, proc, entry_base, entries;
@@ -119,6 +182,7 @@ struct DropPlan {
     uint32_t *bk_list = nullptr, *bk_misc = nullptr;
     int64_t cap_bk = 0;
     int64_t groups_bucketed = 0, groups_sorted = 0;  // groups transposed by each path in the last build
+    TilePlan tile;               // tile.ready: the plan is over image tiles and the arrays above are unused
     int flags = -1;              // PCT_DROP_* flags the plan was built with
     bool desc_all = false;       // desc holds a descriptor for every reconstruction history
     bool ready = false;
@@ -223,6 +287,7 @@ struct pct_ctx {
     int drop_flags = PCT_DROP_SPATIAL_ORDER | PCT_DROP_BRICKS | PCT_DROP_COLS_SLICED;  // PCT_DROP_FLAGS
     int mlp_blocks_per_cu = -1;  // MLP list kernel grid: workgroups per CU, 0 = one lane per history, -1 = auto (PCT_MLP_BLOCKS_PER_CU)
     int drop_pipeline = 1;  // MLP lists of the next transposition groups built while a group is transposed (PCT_DROP_PIPELINE)
+    int drop_tiles = -1;    // DROP over image tiles: -1 by the rule of pct_tiles_prepare, 0 never, 1 wherever the lists fit (PCT_DROP_TILES)
     int64_t drop_group_entries = 1ll << 30;  // list entries per transposition group (PCT_DROP_GROUP_ENTRIES)
     double* accum64 = nullptr;
     float* accum32 = nullptr;
@@ -311,11 +376,19 @@ using MlpLaunch = std::function<int(int64_t h0, int64_t h1, hipStream_t s)>;
 // Builds the DROP plan from the lists.  With `mlp`, the lists are not built yet: the MLP kernel runs
 // group by group on ctx->stream2 while the earlier groups are transposed on ctx->stream.
 int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp = nullptr);
+// The tiles' plan, iterations and residual (k_drop_tiles.hip).  pct_tiles_prepare leaves *done false where
+// the lists do not fit the tiles' packed layout; *lists_built then says whether `mlp` has run over every history.
+bool pct_tiles_wanted(const pct_ctx* ctx);
+int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* lists_built);
+void pct_tile_plan_free(TilePlan* T);
+int pct_tiles_enter(pct_ctx* ctx, bool enter);
+int pct_tiles_iterate(pct_ctx* ctx, int iterations, DropTiming* timing);
+int pct_tiles_residual(pct_ctx* ctx);
 int pct_median_filter_fbp(pct_ctx* ctx);
 int pct_avg_filter_hull(pct_ctx* ctx);
 void pct_drop_plan_free(DropPlan* plan);
 int pct_drop_enter(pct_ctx* ctx, bool enter);  // image into (true) / out of the DROP layout
-int pct_drop_iterate_plan(pct_ctx* ctx, DropTiming* timing);
+int pct_drop_iterate_plan(pct_ctx* ctx, int iterations, DropTiming* timing);
 int pct_stage_residual(pct_ctx* ctx, double* norm);
 // list segments: the segment length in histories (0 = no segments), and the segmented DROP iteration and
 // residual over every segment (segments.hip)

@@ -219,7 +219,7 @@ int pct_stage_drop(pct_ctx* ctx, int iterations, DropTiming* timing)
     if (!ctx->plan.ready || ctx->plan.flags != ctx->drop_flags) PCT_TRY(pct_drop_prepare(ctx));
     if (!ctx->P.tvs_on) {
         PCT_TRY(pct_drop_enter(ctx, true));
-        for (int it = 0; it < iterations; it++) PCT_TRY(pct_drop_iterate_plan(ctx, timing));
+        PCT_TRY(pct_drop_iterate_plan(ctx, iterations, timing));
         PCT_TRY(pct_drop_enter(ctx, false));
         ctx->drop_k += iterations;
         return PCT_OK;
@@ -230,7 +230,7 @@ int pct_stage_drop(pct_ctx* ctx, int iterations, DropTiming* timing)
         const int k = ++ctx->drop_k;
         if (ctx->P.tvs_first) PCT_TRY(pct_tvs_iteration(ctx, k));
         PCT_TRY(pct_drop_enter(ctx, true));
-        PCT_TRY(pct_drop_iterate_plan(ctx, timing));
+        PCT_TRY(pct_drop_iterate_plan(ctx, 1, timing));
         PCT_TRY(pct_drop_enter(ctx, false));
         if (!ctx->P.tvs_first) PCT_TRY(pct_tvs_iteration(ctx, k));
     }

@@ -32,6 +32,7 @@
 #include <hip/hip_ext.h>
 #include <hipcub/hipcub.hpp>
 
+#include "drop_sums.h"
 #include "internal.h"
 
 namespace {
@@ -516,88 +517,6 @@ __global__ void __launch_bounds__(kWave) k_slice_fill(int64_t NS, int64_t chunk,
     }
 }
 
-constexpr int kUnroll = 8;
-
-// Bounds of a nonzero float term of a row sum: |f| < 2^top, and f is a multiple of 2^lsb (its lowest set
-// significand bit).  Zero terms leave the bounds alone.
-__device__ __forceinline__ void term_bounds(float f, int& top, int& lsb)
-{
-    const uint32_t b = __float_as_uint(f) & 0x7fffffffu;
-    if (!b) return;
-    const int ef = (int)(b >> 23);
-    uint32_t m = b & 0x7fffffu;
-    int t, l;
-    if (ef == 0) {  // subnormal: m * 2^-149
-        t = -149 + 32 - __clz(m);
-        l = -149 + __ffs(m) - 1;
-    } else {        // (2^23 + m) * 2^(ef - 150); Inf and NaN (ef = 255) get top 129 and force the ordered sum
-        m |= 0x800000u;
-        t = ef - 126;
-        l = ef - 150 + __ffs(m) - 1;
-    }
-    top = t > top ? t : top;
-    lsb = l < lsb ? l : lsb;
-}
-
-// a_i.x / L_i of one history: the sum of x over its list with the row kernel's lanes and loads
-// (G lanes, kUnroll list loads and then kUnroll gathers in flight per lane, lane l summing entries
-// l, l + G, l + 2G, ... in order, then a butterfly over the G partial sums).  The reference sums the
-// list in order (DS.cu:9245), and the regrouped sum equals the ordered one whenever no partial sum rounds:
-// with every term a multiple of 2^lsb and below 2^top in magnitude, any partial sum of at most cnt terms
-// is a multiple of 2^lsb below 2^(top + ceil(log2 cnt)), exact in double when top + ceil(log2 cnt) - lsb
-// <= 53.  The G lanes of a failing row gather its list again in chunks and all add the chunk in list order
-// from the lanes' registers.  The sum is valid in lane 0.  (Tracking the bounds this way costs about 1 us
-// per DROP block; comparing raw bit patterns instead measured 7 us.)
-template <int G>
-__device__ inline double row_sum(const uint32_t* __restrict__ lst, int cnt, const float* __restrict__ x, int lane)
-{
-    double part = 0.0;
-    int top = -1000, lsb = 1000;
-    for (int j = lane; j < cnt; j += kUnroll * G) {
-        uint32_t a[kUnroll];
-        float xv[kUnroll];
-#pragma unroll
-        for (int q = 0; q < kUnroll; q++) a[q] = j + q * G < cnt ? lst[j + q * G] : 0u;
-#pragma unroll
-        for (int q = 0; q < kUnroll; q++) xv[q] = j + q * G < cnt ? x[a[q]] : 0.0f;
-#pragma unroll
-        for (int q = 0; q < kUnroll; q++)
-            if (j + q * G < cnt) {
-                part += (double)xv[q];
-                term_bounds(xv[q], top, lsb);
-            }
-    }
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) {
-        part += __shfl_xor(part, o, G);
-        const int t = __shfl_xor(top, o, G), l = __shfl_xor(lsb, o, G);
-        top = t > top ? t : top;
-        lsb = l < lsb ? l : lsb;
-    }
-    const int lg = cnt > 1 ? 32 - __clz((uint32_t)cnt - 1u) : 0;  // ceil(log2 cnt)
-    if (top + lg - lsb > 53) {  // the same in the G lanes after the butterfly; all-zero rows (top -1000) never fail
-        // the ordered sum: chunks of kUnroll * G entries gathered as above (entry j + q G + l in lane l), then
-        // added in list order by every lane from the lanes' registers
-        double s = 0.0;
-        for (int j = 0; j < cnt; j += kUnroll * G) {
-            float xv[kUnroll];
-#pragma unroll
-            for (int q = 0; q < kUnroll; q++) {
-                const int e = j + q * G + lane;
-                xv[q] = e < cnt ? x[lst[e]] : 0.0f;
-            }
-#pragma unroll
-            for (int q = 0; q < kUnroll; q++)
-                for (int l = 0; l < G; l++) {
-                    const float v = __shfl(xv[q], l, G);
-                    if (j + q * G + l < cnt) s += (double)v;
-                }
-        }
-        part = s;
-    }
-    return part;
-}
-
 // per history: u_i (DS.cu:9321-9380 with the list of find_MLP_path_GPU_tabulated).
 // G lanes per history (G | 64), histories taken in rank order.
 template <int G>
@@ -612,7 +531,7 @@ __global__ void __launch_bounds__(kBlock) k_drop_rows(int64_t start, int64_t pro
     if (k >= proc) return;  // the G lanes of a history leave together
     const RowDesc d = desc[start + k];
     const int cnt = (int)d.cnt;
-    const double part = row_sum<G>(vox + d.off, cnt, x, lane);
+    const double part = row_sum<G>(vox + d.off, cnt, x, lane, SameIndex{});
     if (lane == 0) {
         const double L = d.chord;
         const double ax = part * L;
@@ -634,7 +553,7 @@ __global__ void __launch_bounds__(kBlock) k_residual(int64_t n, const int64_t* _
     const int64_t stride = (int64_t)gridDim.x * (blockDim.x / G);
     for (int64_t p = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; p < n; p += stride) {
         const int cnt = (int)cnt_arr[p];   // the G lanes of a history loop together
-        const double part = row_sum<G>(vox + off[p], cnt, x, lane);
+        const double part = row_sum<G>(vox + off[p], cnt, x, lane, SameIndex{});
         if (lane == 0) {
             const double r = (double)wepl[p] - chord[p] * part;
             r2[p] = cnt >= min_len ? r * r : 0.0;
@@ -654,40 +573,13 @@ __global__ void __launch_bounds__(kBlock) k_residual_desc(int64_t n, const RowDe
     for (int64_t p = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; p < n; p += stride) {
         const RowDesc d = desc[p];
         const int cnt = (int)d.cnt;
-        const double part = row_sum<G>(vox + d.off, cnt, x, lane);
+        const double part = row_sum<G>(vox + d.off, cnt, x, lane, SameIndex{});
         if (lane == 0) {
             const double r = (double)d.wepl - d.chord * part;
             r2[p] = cnt >= min_len ? r * r : 0.0;
         }
     }
 }
-
-// Running per-voxel sum in history order: FP64 (s = u_1 + u_2 + ...), FP32 (the reference's float
-// sums), or FP32 with Kahan compensation (from s = c = 0).
-template <int ACC>
-struct ColAcc {
-    double s64 = 0.0;
-    float s32 = 0.0f, c32 = 0.0f;
-    bool first = true;
-    __device__ __forceinline__ void add(double rv)
-    {
-        if (ACC == PCT_ACCUM_FP64) {
-            s64 = first ? rv : s64 + rv;
-        } else if (ACC == PCT_ACCUM_FP32) {
-            s32 = first ? (float)rv : s32 + (float)rv;
-        } else {
-            const float y = (float)rv - c32;
-            const float t = s32 + y;
-            c32 = (t - s32) - y;
-            s32 = t;
-        }
-        first = false;
-    }
-    __device__ __forceinline__ float mean(uint32_t n) const
-    {
-        return ACC == PCT_ACCUM_FP64 ? (float)(s64 / (double)n) : s32 / (float)n;
-    }
-};
 
 // Sum of the n = e - b updates of one voxel in history order, divided by n (the voxel's S).
 // The first min(n, K) updates arrive prefetched in rv; the rest are loaded K at a time (K rank
@@ -934,7 +826,8 @@ int build_slices(pct_ctx* ctx, DropPlan& D)
 
 }  // namespace
 
-void pct_drop_plan_free(DropPlan* D)
+// the arrays of the transposed lists
+static void free_lists(DropPlan* D)
 {
     pct_free(&D->t_vox);
     pct_free(&D->t_off);
@@ -973,6 +866,12 @@ void pct_drop_plan_free(DropPlan* D)
     D->cap_vox_b = D->cap_x_b = 0;
     D->vox_b_ready = false;
     D->cap_entries = D->cap_off = D->cap_r = D->cap_perm = D->cap_group_e = D->cap_group_h = D->cap_group_b = 0;
+}
+
+void pct_drop_plan_free(DropPlan* D)
+{
+    free_lists(D);
+    pct_tile_plan_free(&D->tile);
     D->ready = false;
 }
 
@@ -1051,9 +950,20 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
     const pct_params& P = ctx->P;
     hipStream_t s = ctx->stream;
     const int64_t n = ctx->n_recon;
+    DropPlan& D = ctx->plan;
+    if (pct_tiles_wanted(ctx)) {
+        D.ready = false;
+        bool done = false, built = false;
+        PCT_TRY(pct_tiles_prepare(ctx, mlp, &done, &built));
+        if (done) {
+            free_lists(&D);  // of an earlier plan with other flags
+            return PCT_OK;
+        }
+        if (built) mlp = nullptr;  // the lists exist now
+    }
+    pct_tile_plan_free(&D.tile);
     const bool pipe = mlp != nullptr;  // the lists are built group by group below
     const int64_t BS = P.drop_block_size;
-    DropPlan& D = ctx->plan;
     D.blocks.clear();
     D.groups.clear();
     D.ready = false;
@@ -1466,6 +1376,7 @@ void drop_launch(K kernel, dim3 g, dim3 b, hipStream_t s, std::vector<hipEvent_t
 int pct_drop_enter(pct_ctx* ctx, bool enter)
 {
     const DropPlan& D = ctx->plan;
+    if (D.tile.ready) return pct_tiles_enter(ctx, enter);
     if (!(D.flags & PCT_DROP_BRICKS)) return PCT_OK;
     const pct_params& P = ctx->P;
     const BrickGeom bg{(uint32_t)P.columns, (uint32_t)P.rows, (uint32_t)D.nbx, (uint32_t)D.nby};
@@ -1475,8 +1386,17 @@ int pct_drop_enter(pct_ctx* ctx, bool enter)
     return PCT_OK;
 }
 
-// One DROP iteration with the prepared plan; optional per-kernel timing.
-int pct_drop_iterate_plan(pct_ctx* ctx, DropTiming* timing)
+static int iterate_once(pct_ctx* ctx, DropTiming* timing);
+
+// `iterations` DROP iterations with the prepared plan; optional per-kernel timing.
+int pct_drop_iterate_plan(pct_ctx* ctx, int iterations, DropTiming* timing)
+{
+    if (ctx->plan.tile.ready) return pct_tiles_iterate(ctx, iterations, timing);
+    for (int it = 0; it < iterations; it++) PCT_TRY(iterate_once(ctx, timing));
+    return PCT_OK;
+}
+
+static int iterate_once(pct_ctx* ctx, DropTiming* timing)
 {
     const pct_params& P = ctx->P;
     hipStream_t s = ctx->stream;
@@ -1596,7 +1516,8 @@ int pct_stage_residual(pct_ctx* ctx, double* norm)
     if (n > 0) {
         const uint32_t* vox = ctx->list_vox;
         const float* x = ctx->x;
-        if (D.ready && (D.flags & PCT_DROP_BRICKS) && D.vox_b_ready && D.x_b) {
+        const bool tiles = D.ready && D.tile.ready && D.desc_all;
+        if (!tiles && D.ready && !D.tile.ready && (D.flags & PCT_DROP_BRICKS) && D.vox_b_ready && D.x_b) {
             const pct_params& P = ctx->P;
             const BrickGeom bg{(uint32_t)P.columns, (uint32_t)P.rows, (uint32_t)D.nbx, (uint32_t)D.nby};
             hipLaunchKernelGGL(k_x_bricks, dim3(grid_for(P.num_voxels)), dim3(kBlock), 0, s, (int64_t)P.num_voxels,
@@ -1606,7 +1527,9 @@ int pct_stage_residual(pct_ctx* ctx, double* norm)
         }
         constexpr int G = 16;
         const unsigned rg = pct_grid_capped(n * G, kBlock, 1u << 20);  // grid-stride kernels
-        if (vox == D.vox_b && D.desc_all)  // the plan's descriptors cover every history
+        if (tiles)
+            PCT_TRY(pct_tiles_residual(ctx));
+        else if (vox == D.vox_b && D.desc_all)  // the plan's descriptors cover every history
             hipLaunchKernelGGL(k_residual_desc<G>, dim3(rg), dim3(kBlock), 0, s, n, D.desc, vox, x,
                                ctx->P.min_mlp_length, ctx->res_r2);
         else

@@ -729,6 +729,7 @@ int pct_stage_build_lists(pct_ctx* ctx)
         PCT_TRY(pct_alloc(ctx, &ctx->list_vox, total));
         ctx->list_cap = total;
     }
+    ctx->list_slots = total;
     ctx->plan.vox_b_ready = false;  // the brick copy of the lists belongs to the previous build
     const size_t lds = (size_t)a.n_steps * 6 * sizeof(double);
     if (lds > 64 * 1024) {
@@ -807,7 +808,6 @@ int pct_stage_build_lists(pct_ctx* ctx)
     PCT_CHECK_HIP(ctx, hipMemcpyAsync(&listed, d_total, sizeof(listed), hipMemcpyDeviceToHost, s));
     PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
     ctx->list_entries = (int64_t)listed;
-    ctx->list_slots = total;
     ctx->stage = ST_LISTS;
     if (pipe) return PCT_OK;  // the plan was built with the lists
     // the DROP blocks' transposed lists belong to the list build

@@ -114,7 +114,7 @@ int drop_iteration_segments(pct_ctx* ctx, int64_t seg, DropTiming* timing)
         PCT_TRY(plan_totals(ctx, &st, timing != nullptr));
         t0 = std::chrono::steady_clock::now();
         PCT_TRY(pct_drop_enter(ctx, true));
-        PCT_TRY(pct_drop_iterate_plan(ctx, timing));
+        PCT_TRY(pct_drop_iterate_plan(ctx, 1, timing));
         PCT_TRY(pct_drop_enter(ctx, false));
         PCT_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
         st.drop_ms += ms_since(t0);
