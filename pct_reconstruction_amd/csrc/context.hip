@@ -120,7 +120,14 @@ int pct_ctx_create(const pct_params* p, int device, pct_ctx** out)
     // hull carving: LDS hash slots of the fused walk, or 0 for one walk per method (the counts are the same)
     if (const char* e = std::getenv("PCT_CARVE_TABLE")) {
         int t = std::atoi(e);
-        if (t == 0 || t == 4096 || t == 8192 || t == 16384) ctx->carve_table = t;
+        if (t == 0 || t == 4096 || t == 8192 || t == 16384) {
+            ctx->carve_table = t;
+            ctx->carve_tiles = 0;
+        }
+    }
+    if (const char* e = std::getenv("PCT_CARVE_TILES")) {
+        int t = std::atoi(e);
+        if (t >= -1 && t <= 1) ctx->carve_tiles = t;
     }
     if (const char* e = std::getenv("PCT_CARVE_BLOCK")) {
         int t = std::atoi(e);
@@ -185,6 +192,7 @@ int pct_ctx_destroy(pct_ctx* ctx)
     pct_free(&ctx->T.p26); pct_free(&ctx->T.p312); pct_free(&ctx->T.step_terms);
     pct_free(&ctx->accum64); pct_free(&ctx->accum32); pct_free(&ctx->S); pct_free(&ctx->touched);
     pct_free(&ctx->n_touched); pct_free(&ctx->list_overflow);
+    pct_carve_free(ctx);
     pct_drop_plan_free(&ctx->plan);
     pct_free(&ctx->tvs_G); pct_free(&ctx->tvs_part); pct_free(&ctx->tvs_res);
     if (ctx->tvs_res_h) (void)hipHostFree(ctx->tvs_res_h);
@@ -651,6 +659,15 @@ int pct_drop_iteration_device(int64_t n, const int64_t* offsets, const uint32_t*
 }
 
 }  // extern "C"
+
+int pct_grow_cub(pct_ctx* ctx, size_t need)
+{
+    if (need <= ctx->cub_tmp_bytes) return PCT_OK;
+    ctx->cub_tmp_bytes = 0;
+    PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, need));
+    ctx->cub_tmp_bytes = need;
+    return PCT_OK;
+}
 
 // unit conversion of freshly loaded raw data (k_preproc.hip has the kernel)
 int pct_launch_units(hipStream_t s, int64_t n, float* const raw[14], int mm, double ts, double us, double vs);

@@ -200,6 +200,19 @@ struct SegStats {
     double lists_ms = 0, drop_ms = 0;  // host wall time in the list builds (incl. plans) and in the DROP blocks
 };
 
+// The hull carving by tiles (k_hull.hip).
+struct alignas(32) CarveRec {  // one history in visiting order
+    float xe, ye, ze, xx, yx, zx;
+    uint32_t inc;  // MSC | SM << 15 | SC << 30
+    float pad;
+};
+struct CarveScratch {  // kept until the reconstruction volume is complete; bounded by a batch of histories
+    CarveRec* recs = nullptr;
+    uint32_t *cap = nullptr, *off = nullptr, *keys = nullptr, *tiles = nullptr;
+    uint64_t* vals = nullptr;
+    int64_t cap_recs = 0, cap_cap = 0, cap_off = 0, cap_keys = 0, cap_tiles = 0, cap_vals = 0;
+};
+
 struct pct_ctx {
     pct_params P;
     int device = 0;
@@ -239,6 +252,8 @@ struct pct_ctx {
     int64_t bin_perm_n = -1;  // u32_d holds the bin order of the first bin_perm_n histories (pct_bin_order)
     int carve_spill = 512;    // LDS count at which a carve visit goes to global memory, 1..512 (PCT_CARVE_SPILL)
     int carve_table = 8192;   // LDS hash slots of the fused carve (4096, 8192, 16384); 0: one walk per method (PCT_CARVE_TABLE)
+    int carve_tiles = -1;      // hull carving by tiles: -1 by rule, 0 never, 1 always (PCT_CARVE_TILES)
+    CarveScratch carve;
     int carve_line_order = 1;  // hull carving in chord-line order (both directions of a line together; PCT_CARVE_LINES)
     int endpoint_order = 1;   // MLP endpoints in sinogram-bin order (PCT_ENDPOINT_ORDER)
     int carve_block = 512;    // lanes per workgroup of the fused carve (256, 512; PCT_CARVE_BLOCK)
@@ -350,6 +365,8 @@ struct pct_tmp {
 };
 
 DevGeom pct_geom(const pct_params& P);
+void pct_carve_free(pct_ctx* ctx);              // the carve's scratch
+int pct_grow_cub(pct_ctx* ctx, size_t need);  // library scratch of at least `need` bytes
 
 // host-side tables (tables.cpp)
 struct HostTables {

@@ -904,15 +904,6 @@ int grow(pct_ctx* ctx, T** p, int64_t* cap, int64_t need)
     *cap = need;
     return PCT_OK;
 }
-int grow_cub(pct_ctx* ctx, size_t need)
-{
-    if (need <= ctx->cub_tmp_bytes) return PCT_OK;
-    ctx->cub_tmp_bytes = 0;
-    PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, need));
-    ctx->cub_tmp_bytes = need;
-    return PCT_OK;
-}
-
 // The segments, tiles and lists of one group (its MLP lists exist).  *fits is false when a tile exceeds the
 // limits of the packed lists.
 int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int bin_bits, BlockTotals* totals, bool* fits)
@@ -933,7 +924,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
     PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, need, W.hkey, W.hkey + H, W.hidx, order, (int)H, 0,
                                                           hbits, s));
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, t, W.nseg, W.q0, (int)(H + 1), s));
-    PCT_TRY(grow_cub(ctx, std::max(need, t)));
+    PCT_TRY(pct_grow_cub(ctx, std::max(need, t)));
     // visiting order and the histories' segments
     hipLaunchKernelGGL(k_tile_hist_keys, dim3(grid_for(H)), dim3(kBlock), 0, s, a.h0, H, a.BS, a.rb0, a.proc_raw,
                        ctx->bin_num, bin_bits, W.hkey, W.hidx);
@@ -972,7 +963,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
                                                           0, kbits, s));
     PCT_CHECK_HIP(ctx, hipcub::DeviceRunLengthEncode::Encode(nullptr, t, keys_sorted, W.keys, W.runs, W.n_runs, (int)Q, s));
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, t2, W.runs, run_start, (int)Q, s));
-    PCT_TRY(grow_cub(ctx, std::max(need, std::max(t, t2))));
+    PCT_TRY(pct_grow_cub(ctx, std::max(need, std::max(t, t2))));
     hipLaunchKernelGGL(k_tile_cut<true>, dim3(cg), dim3(kBlock), 0, s, a, (uint32_t*)nullptr, W.q0, T.rows, W.keys,
                        W.idx, recs);
     tb = ctx->cub_tmp_bytes;
@@ -1004,7 +995,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
     PCT_CHECK_HIP(ctx, hipcub::DeviceReduce::Max(nullptr, need, W.runs, W.limits + 1, (int)nr, s));
     PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, t, W.need, need_sorted, W.need + 2 * (size_t)nr, by_need,
                                                           (int)nr, 0, 8, s));
-    PCT_TRY(grow_cub(ctx, std::max(need, t)));
+    PCT_TRY(pct_grow_cub(ctx, std::max(need, t)));
     tb = ctx->cub_tmp_bytes;
     PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->cub_tmp, tb, W.need, need_sorted, W.need + 2 * (size_t)nr,
                                                           by_need, (int)nr, 0, 8, s));

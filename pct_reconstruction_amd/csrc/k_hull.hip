@@ -6,8 +6,12 @@
 // reference's bool image); the hull is the cylinder mask without the carved bits.  MSC/SM count
 // traversals with 32-bit integer atomics, which are exact and order independent.  By default one walk
 // serves every method, the histories in sinogram-bin order, with the visits of a workgroup summed in
-// LDS first (k_carve_all); 3.4x faster than one walk per method on the head-50M workload.
+// LDS first: in a hash table (k_carve_all; 3.4x faster than one walk per method on the head-50M workload), or, for MSC and
+// SM counts from 2^18 histories on, in the counts of an image tile that the chords pass through (k_carve_tiles).
+#include <hipcub/hipcub.hpp>
+
 #include "internal.h"
+#include "walk.h"
 
 namespace {
 
@@ -221,6 +225,257 @@ __global__ void __launch_bounds__(BLOCK) k_carve_all(int64_t n, const uint32_t* 
     }
 }
 
+// ---------------------------------------------------------------- carving by tiles ----
+// Counting in LDS needs many visits per voxel and workgroup, and the chords of a workgroup share few voxels when
+// bins hold few histories: with 16M head histories the hash table of k_carve_all overflows, and 21 of its 55 ms went
+// to visits that missed it, 9 to its flush and 12 to its probes.  Here the image is cut into tiles of 64 x 64 x 2
+// voxels, 32 KB of packed counts.  A walk (k_carve_cut) finds where each chord enters a tile, the entries are sorted
+// by tile, and a workgroup takes a chunk of one tile's entries (k_carve_tiles), walks each chord on inside the tile
+// and adds the tile's counts to memory once: no visit needs a probe, a returned value or a global atomic.  The walk
+// is taken twice, but is cheaper (walk.h: 8.9 ms for the cut, 12 before), and both are bound by its FP64 arithmetic.
+// 16M histories, 256 x 256 x 48: gather 2.0, cut 8.9, sort 0.7, tiles 6.7 ms, 18.5 in all (54.6 before); 6M: 6.5
+// (29.8).
+constexpr int kCT = 64, kCTZ = 2, kCTVox = kCT * kCT * kCTZ;
+constexpr int kCarveBlock = 512;
+
+__device__ __forceinline__ uint32_t carve_tile(int vx, int vy, int vz, int ntx, int nty)
+{
+    return ((uint32_t)(vz >> 1) * nty + (uint32_t)(vy >> 6)) * ntx + (uint32_t)(vx >> 6);
+}
+
+__device__ __forceinline__ void chord_line(const CarveRec& r, Walk3& w)
+{
+    w.xs = r.xe;
+    w.ys = r.ye;
+    w.zs = r.ze;
+    w.xm = (r.xe <= r.xx) - (r.xe >= r.xx);
+    w.ym = (r.ye <= r.yx) - (r.ye >= r.yx);
+    w.zm = (r.ze <= r.zx) - (r.ze >= r.zx);
+    w.dy_dx = (double)((r.yx - r.ye) / (r.xx - r.xe));
+    w.dz_dx = (double)((r.zx - r.ze) / (r.xx - r.xe));
+    w.dz_dy = (double)((r.zx - r.ze) / (r.yx - r.ye));
+    w.dx_dy = (double)((r.xx - r.xe) / (r.yx - r.ye));
+    w.dx_dz = (double)((r.xx - r.xe) / (r.zx - r.ze));
+    w.dy_dz = (double)((r.yx - r.ye) / (r.zx - r.ze));
+}
+
+// The histories of a batch in visiting order, and how many tile entries each may have: one more than the tile steps
+// between its first and last voxel, and one for a start on a tile's far edge; none when no method takes it.  cap[n] is
+// 0: the scan's total.
+__global__ void k_carve_gather(int64_t n, const uint32_t* __restrict__ perm, DevGeom g, HistPtrs hp, Gates gt,
+                               CarveRec* __restrict__ recs, uint32_t* __restrict__ cap)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == n) cap[t] = 0;
+    if (t >= n) return;
+    const int64_t i = perm[t];
+    const float w = hp.wepl[i];
+    CarveRec r{hp.xe[i], hp.ye[i], hp.ze[i], hp.xx[i], hp.yx[i], hp.zx[i], 0u, 0.0f};
+    if (gt.msc && w <= gt.msc_hi && w >= gt.msc_lo) r.inc |= 1u;
+    if (gt.sm && w >= gt.sm_lo) r.inc |= 1u << 15;
+    if (gt.sc && w <= gt.sc_hi && w >= gt.sc_lo) r.inc |= 1u << 30;
+    recs[t] = r;
+    uint32_t c = 0;
+    if (r.inc) {
+        auto tiles = [](int a, int b, int n, int shift) {
+            return abs((min(max(b, 0), n) >> shift) - (min(max(a, 0), n) >> shift));
+        };
+        c = (uint32_t)(2 + tiles(pct_calc_voxel(g.X0, r.xe, g.VW), pct_calc_voxel(g.X0, r.xx, g.VW), g.C, 6) +
+                       tiles(pct_calc_voxel(g.Y0, r.ye, g.VH), pct_calc_voxel(g.Y0, r.yx, g.VH), g.R, 6) +
+                       tiles(pct_calc_voxel(g.Z0, r.ze, g.VT), pct_calc_voxel(g.Z0, r.zx, g.VT), g.S, 1));
+    }
+    cap[t] = c;
+}
+
+// The walk of every chord, one entry per tile it passes: key tile, value history | state << 32 (voxel in the tile
+// 13 bits, axis 2 bits (3: the start), full 3 bits, visits 14 bits).  What the tile walk does not take is counted
+// here with global atomics: chords without a z slope (the 2D walk), what follows once the z voxel was clamped or a
+// step left the voxel as it was (voxels can come twice there: an entry's visits are distinct), and what finds no
+// room.  Unused room gets the key n_tiles.
+__global__ void __launch_bounds__(256) k_carve_cut(int64_t n, DevGeom g, const CarveRec* __restrict__ recs,
+                                                   const uint32_t* __restrict__ off, int ntx, int nty, uint32_t n_tiles,
+                                                   uint32_t* __restrict__ keys, uint64_t* __restrict__ vals,
+                                                   uint32_t* __restrict__ carved, int32_t* __restrict__ msc_counts,
+                                                   int32_t* __restrict__ sm_counts)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const CarveRec r = recs[t];
+    uint32_t q = off[t];
+    const uint32_t end = off[t + 1];
+    auto count = [&](int64_t v) {
+        if (r.inc >> 30) atomicOr(&carved[v >> 5], 1u << (v & 31));
+        if (r.inc & 1u) atomicAdd(&msc_counts[v], 1);
+        if (r.inc & (1u << 15)) atomicAdd(&sm_counts[v], 1);
+    };
+    if (r.inc) {
+        Walk3 w;
+        chord_line(r, w);
+        if (w.zm == 0) {
+            carve_walk(g, r.xe, r.ye, r.ze, r.xx, r.yx, r.zx, count);
+        } else {
+            w.vx = pct_calc_voxel(g.X0, r.xe, g.VW);
+            w.vy = pct_calc_voxel(g.Y0, r.ye, g.VH);
+            w.vz = pct_calc_voxel(g.Z0, r.ze, g.VT);
+            const int ox = pct_calc_voxel(g.X0, r.xx, g.VW), oy = pct_calc_voxel(g.Y0, r.yx, g.VH),
+                      oz = pct_calc_voxel(g.Z0, r.zx, g.VT);
+            const int64_t out = ox + (int64_t)oy * g.C + (int64_t)oz * g.C * g.R;
+            const int none = -1;  // no voxel of the image: image addresses have 31 bits
+            const int at_out = out >= 0 && out < g.NV ? (int)out : none;
+            w.ax = w.xm;
+            w.ay = -w.ym * g.C;
+            w.az = -w.zm * g.C * g.R;
+            auto address = [&] { return w.vx + (w.vy + w.vz * g.R) * g.C; };
+            auto ended = [&] {
+                return w.at == at_out || (uint32_t)w.vx >= (uint32_t)g.C || (uint32_t)w.vy >= (uint32_t)g.R || w.vz >= g.S;
+            };
+            // a start outside the image has no address
+            bool end_walk = (uint32_t)w.vx >= (uint32_t)g.C || (uint32_t)w.vy >= (uint32_t)g.R ||
+                            (uint32_t)w.vz >= (uint32_t)g.S;
+            w.at = end_walk ? none : address();
+            end_walk = end_walk || w.at == at_out;
+            w.begin(g);
+            int tx = w.vx, ty = w.vy, tz = w.vz;  // where the entry began
+            uint32_t state = 3u << 13, visits = 0;
+            bool direct = q == end;
+            auto flush = [&] {
+                if (visits) {
+                    keys[q] = carve_tile(tx, ty, tz, ntx, nty);
+                    vals[q++] = (uint64_t)t | (uint64_t)(state | visits << 18 | (tz & 1) << 12 | (ty & 63) << 6 |
+                                                         (tx & 63)) << 32;
+                    visits = 0;
+                }
+            };
+            const int cap = 4 * (g.C + g.R + g.S) + 16;
+            int steps = 0;
+            while (!end_walk) {
+                if (direct) count(w.at);
+                else visits++;
+                int full;
+                bool clamped;
+                const int last = w.at, axis = w.step(g, &full, &clamped);
+                if (clamped) w.at = address();
+                end_walk = ended() || ++steps > cap;
+                if (clamped || w.at == last || ((w.vx ^ tx) | (w.vy ^ ty)) >> 6 || (w.vz ^ tz) >> 1) {
+                    flush();
+                    direct = direct || clamped || w.at == last || q == end;
+                    tx = w.vx;
+                    ty = w.vy;
+                    tz = w.vz;
+                    state = (uint32_t)(axis << 13 | full << 15);
+                }
+            }
+            flush();
+        }
+    }
+    for (; q < end; q++) {
+        keys[q] = n_tiles;
+        vals[q] = 0;
+    }
+}
+
+// start[t]: first sorted entry of tile t; first_chunk[t]: the chunks of the tiles before t
+__global__ void __launch_bounds__(1024) k_carve_chunks(uint32_t n_tiles, uint32_t n, uint32_t chunk,
+                                                       const uint32_t* __restrict__ keys, uint32_t* __restrict__ start,
+                                                       uint32_t* __restrict__ first_chunk)
+{
+    __shared__ uint32_t part[1024], total;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    for (uint32_t t0 = 0; t0 <= n_tiles; t0 += 1024) {
+        const uint32_t t = t0 + threadIdx.x;
+        auto find = [&](uint32_t key) {
+            uint32_t lo = 0, hi = n;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                if (keys[mid] < key) lo = mid + 1;
+                else hi = mid;
+            }
+            return lo;
+        };
+        uint32_t mine = 0;
+        if (t <= n_tiles) {
+            const uint32_t a = find(t);
+            start[t] = a;
+            if (t < n_tiles) mine = (find(t + 1) - a + chunk - 1) / chunk;
+        }
+        part[threadIdx.x] = mine;
+        __syncthreads();
+        for (uint32_t o = 1; o < 1024; o <<= 1) {
+            const uint32_t y = threadIdx.x >= o ? part[threadIdx.x - o] : 0u;
+            __syncthreads();
+            part[threadIdx.x] += y;
+            __syncthreads();
+        }
+        if (t <= n_tiles) first_chunk[t] = total + part[threadIdx.x] - mine;
+        __syncthreads();
+        if (threadIdx.x == 1023) total += part[1023];
+        __syncthreads();
+    }
+}
+
+// A chunk of one tile's entries per workgroup: a chord visits a voxel of the tile once (the walk is monotone up to
+// a clamp), so a field of 15 bits holds the counts of up to 32767 entries.
+__global__ void __launch_bounds__(kCarveBlock) k_carve_tiles(DevGeom g, const CarveRec* __restrict__ recs,
+                                                             const uint64_t* __restrict__ vals, uint32_t n_tiles,
+                                                             uint32_t chunk, const uint32_t* __restrict__ start,
+                                                             const uint32_t* __restrict__ first_chunk, int ntx, int nty,
+                                                             uint32_t* __restrict__ carved,
+                                                             int32_t* __restrict__ msc_counts,
+                                                             int32_t* __restrict__ sm_counts)
+{
+    __shared__ uint32_t cnt[kCTVox];
+    const uint32_t b = blockIdx.x;
+    if (b >= first_chunk[n_tiles]) return;
+    uint32_t lo = 0, hi = n_tiles;  // first_chunk[lo] <= b < first_chunk[hi]
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (first_chunk[mid] <= b) lo = mid;
+        else hi = mid;
+    }
+    const uint32_t tile = lo, e0 = start[tile] + (b - first_chunk[tile]) * chunk;
+    const uint32_t e1 = min(e0 + chunk, start[tile + 1]);
+    const int bx = (int)(tile % (uint32_t)ntx) * kCT, by = (int)(tile / (uint32_t)ntx % (uint32_t)nty) * kCT,
+              bz = (int)(tile / ((uint32_t)ntx * nty)) * kCTZ;
+    for (uint32_t k = threadIdx.x; k < (uint32_t)kCTVox; k += kCarveBlock) cnt[k] = 0u;
+    __syncthreads();
+    for (uint32_t e = e0 + threadIdx.x; e < e1; e += kCarveBlock) {
+        const uint64_t v = vals[e];
+        const CarveRec r = recs[(uint32_t)v];
+        const uint32_t s = (uint32_t)(v >> 32);
+        Walk3 w;
+        chord_line(r, w);
+        w.vx = bx + (int)(s & 63u);
+        w.vy = by + (int)((s >> 6) & 63u);
+        w.vz = bz + (int)((s >> 12) & 1u);
+        const int axis = (int)(s >> 13) & 3, full = (int)(s >> 15) & 7;
+        if (axis == 3) w.begin(g);
+        else w.resume(g, axis, full);
+        w.ax = w.xm;
+        w.ay = -w.ym * 64;
+        w.az = -w.zm * 4096;
+        w.at = (int)(s & 8191u);
+        for (uint32_t visits = s >> 18;;) {
+            if (r.inc & 0x3fffffffu) atomicAdd(&cnt[w.at], r.inc & 0x3fffffffu);
+            if (r.inc >> 30) atomicOr(&cnt[w.at], 1u << 30);
+            if (--visits == 0) break;
+            int f;
+            bool clamped;
+            w.step(g, &f, &clamped);
+        }
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < (uint32_t)kCTVox; k += kCarveBlock) {
+        const uint32_t n = cnt[k];
+        if (!n) continue;
+        const int64_t v = (bx + (int64_t)(k & 63u)) + (by + (int64_t)((k >> 6) & 63u)) * g.C +
+                          (bz + (int64_t)(k >> 12)) * g.C * g.R;
+        if (n >> 30) atomicOr(&carved[v >> 5], 1u << (v & 31));
+        if (n & 0x7fffu) atomicAdd(&msc_counts[v], (int32_t)(n & 0x7fffu));
+        if ((n >> 15) & 0x7fffu) atomicAdd(&sm_counts[v], (int32_t)((n >> 15) & 0x7fffu));
+    }
+}
+
 // SC hull = cylinder mask without the carved voxels
 __global__ void k_sc_finish(DevGeom g, const uint32_t* carved, uint8_t* hull)
 {
@@ -352,6 +607,109 @@ DevGeom pct_geom(const pct_params& P)
     return g;
 }
 
+namespace {
+
+// Histories from which the counts of MSC and SM go by tiles.  Preprocessing on a 256 x 256 head grid, table / tiles:
+// 0.25M histories 4.1 / 3.0 ms, 2M 20 / 11, 16M 73 / 40; on a 90 x 74 grid 0.15M 1.19 / 1.25 (3.38 / 3.57 in a new
+// context, which allocates the scratch), 0.3M 1.63 / 1.53.  SC alone keeps the table at any size: its gate takes few
+// histories, and a visit that misses only sets a bit (2M histories on a 200 x 200 cylinder grid, a whole
+// reconstruction: 65.3 ms by table, 66.0 by tiles).
+constexpr int64_t kCarveTilesMin = 1 << 18;
+
+void carve_tiles_free(CarveScratch& W)
+{
+    pct_free(&W.recs);
+    pct_free(&W.cap);
+    pct_free(&W.off);
+    pct_free(&W.keys);
+    pct_free(&W.vals);
+    pct_free(&W.tiles);
+    W = CarveScratch{};
+}
+
+// The counts by tiles, in batches of histories (in visiting order ctx->u32_d).  *done: the histories counted; fewer
+// than n, with PCT_OK, where there was no memory for the rest.
+int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gates& gt, int64_t n, int64_t* done)
+{
+    hipStream_t s = ctx->stream;
+    CarveScratch& W = ctx->carve;
+    const int ntx = (g.C + kCT - 1) / kCT, nty = (g.R + kCT - 1) / kCT, ntz = (g.S + kCTZ - 1) / kCTZ;
+    const int64_t tiles = (int64_t)ntx * nty * ntz;
+    const uint32_t n_tiles = (uint32_t)tiles;
+    // 4M histories (0.9 GB on the 256 x 256 head grid), fewer where a chord may pass very many tiles
+    const int64_t kBatch = std::min<int64_t>(4 << 20, (int64_t)(1 << 28) / (2 + ntx + nty + ntz));
+    int bits = 1;
+    while ((1ll << bits) < tiles + 1) bits++;
+    auto grow = [&](auto** p, int64_t* cap, int64_t need) -> int {
+        if (need <= *cap) return PCT_OK;
+        *cap = 0;
+        PCT_TRY(pct_alloc(ctx, p, need));
+        *cap = need;
+        return PCT_OK;
+    };
+    auto no_memory = [&](int rc) {
+        if (rc != PCT_E_NOMEM) return rc;
+        (void)hipGetLastError();
+        ctx->err.clear();
+        carve_tiles_free(W);
+        return (int)PCT_OK;
+    };
+    for (*done = 0; *done < n;) {
+        const int64_t m = std::min(kBatch, n - *done);
+        size_t scan = 0, sort = 0;
+        int rc = grow(&W.recs, &W.cap_recs, m);
+        if (rc == PCT_OK) rc = grow(&W.cap, &W.cap_cap, m + 1);
+        if (rc == PCT_OK) rc = grow(&W.off, &W.cap_off, m + 1);
+        if (rc == PCT_OK) rc = grow(&W.tiles, &W.cap_tiles, 2 * (tiles + 1));
+        if (rc != PCT_OK) return no_memory(rc);
+        PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, scan, W.cap, W.off, (int)(m + 1), s));
+        rc = pct_grow_cub(ctx, scan);
+        if (rc != PCT_OK) return no_memory(rc);
+        hipLaunchKernelGGL(k_carve_gather, dim3(grid_for(m + 1)), dim3(kBlock), 0, s, m, ctx->u32_d + *done, g, hp, gt,
+                           W.recs, W.cap);
+        scan = ctx->cub_tmp_bytes;
+        PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, scan, W.cap, W.off, (int)(m + 1), s));
+        uint32_t total = 0;
+        PCT_CHECK_HIP(ctx, hipMemcpyAsync(&total, W.off + m, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+        if (total > 0) {
+            uint32_t *keys, *sorted_keys, *start = W.tiles, *first_chunk = W.tiles + tiles + 1;
+            uint64_t *vals, *sorted_vals;
+            const int64_t room = 2 * ((int64_t)total + total / 16);
+            rc = grow(&W.keys, &W.cap_keys, room);
+            if (rc == PCT_OK) rc = grow(&W.vals, &W.cap_vals, room);
+            if (rc != PCT_OK) return no_memory(rc);
+            keys = W.keys;
+            sorted_keys = keys + total;
+            vals = W.vals;
+            sorted_vals = vals + total;
+            PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, sort, keys, sorted_keys, vals, sorted_vals,
+                                                                  (int)total, 0, bits, s));
+            rc = pct_grow_cub(ctx, sort);
+            if (rc != PCT_OK) return no_memory(rc);
+            sort = ctx->cub_tmp_bytes;
+            hipLaunchKernelGGL(k_carve_cut, dim3(pct_grid_for(m, 256)), dim3(256), 0, s, m, g, W.recs, W.off, ntx, nty,
+                               n_tiles, keys, vals, ctx->sc_carved, ctx->msc_counts, ctx->sm_counts);
+            PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->cub_tmp, sort, keys, sorted_keys, vals,
+                                                                  sorted_vals, (int)total, 0, bits, s));
+            // several thousand workgroups where there is work for them; 15-bit counts
+            const uint32_t chunk = std::min(32767u, std::max(2048u, total / 4096u));
+            hipLaunchKernelGGL(k_carve_chunks, dim3(1), dim3(1024), 0, s, n_tiles, total, chunk, sorted_keys, start,
+                               first_chunk);
+            hipLaunchKernelGGL(k_carve_tiles, dim3(total / chunk + n_tiles + 1), dim3(kCarveBlock), 0, s, g, W.recs,
+                               sorted_vals, n_tiles, chunk, start, first_chunk, ntx, nty, ctx->sc_carved,
+                               ctx->msc_counts, ctx->sm_counts);
+            PCT_CHECK_HIP(ctx, hipGetLastError());
+        }
+        *done += m;
+    }
+    return PCT_OK;
+}
+
+}  // namespace
+
+void pct_carve_free(pct_ctx* ctx) { carve_tiles_free(ctx->carve); }
+
 // hull_initializations (DS.cu:6636) + the carving counts of hull_detection (:6607)
 int pct_carve_counts(pct_ctx* ctx)
 {
@@ -377,15 +735,20 @@ int pct_carve_counts(pct_ctx* ctx)
         if (ctx->carve_table && NV < (int64_t)kEmpty && n <= 0x7fffffff) {
             // histories in sinogram-bin order (a sort of up to 2^31 - 1); voxel numbers are 32-bit table keys
             // below kEmpty
-            PCT_TRY(ctx->carve_line_order ? pct_line_order(ctx, n) : pct_bin_order(ctx, n));
+            const bool worth = (P.msc_on || P.sm_on) && n >= kCarveTilesMin;
+            const bool tiles = (ctx->carve_tiles == 1 || (ctx->carve_tiles < 0 && worth)) && NV <= 0x7fffffff;
+            PCT_TRY(ctx->carve_line_order && !tiles ? pct_line_order(ctx, n) : pct_bin_order(ctx, n));
             Gates gt{P.sc_on, P.msc_on, P.sm_on, P.sc_lower_threshold, P.sc_upper_threshold, P.msc_lower_threshold,
                      P.msc_upper_threshold, P.sm_lower_threshold, (uint32_t)ctx->carve_spill};
+            int64_t done = 0;
+            if (tiles) PCT_TRY(carve_by_tiles(ctx, g, hp, gt, n, &done));
             const int tb = ctx->carve_table, bs = ctx->carve_block;
             auto kern = tb == 4096    ? (bs == 512 ? k_carve_all<4096, 512> : k_carve_all<4096, 256>)
                         : tb == 16384 ? (bs == 512 ? k_carve_all<16384, 512> : k_carve_all<16384, 256>)
                                       : (bs == 512 ? k_carve_all<8192, 512> : k_carve_all<8192, 256>);
-            hipLaunchKernelGGL(kern, dim3(grid_for(n, bs)), dim3(bs), 0, s, n, ctx->u32_d, g, hp, gt,
-                               ctx->sc_carved, ctx->msc_counts, ctx->sm_counts);
+            if (done < n)
+                hipLaunchKernelGGL(kern, dim3(grid_for(n - done, bs)), dim3(bs), 0, s, n - done, ctx->u32_d + done, g, hp,
+                                   gt, ctx->sc_carved, ctx->msc_counts, ctx->sm_counts);
         } else {
             if (P.sc_on)
                 hipLaunchKernelGGL(k_carve, dim3(grid_for(n)), dim3(kBlock), 0, s, n, g, hp, 0, P.sc_lower_threshold,

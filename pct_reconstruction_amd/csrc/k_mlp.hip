@@ -607,6 +607,7 @@ int pct_stage_endpoints(pct_ctx* ctx)
     hipStream_t s = ctx->stream;
     const int64_t n = ctx->n_hist;
     DevGeom g = pct_geom(P);
+    pct_carve_free(ctx);  // the lists size themselves by the free memory
     H10 hp;
     for (int k = 0; k < 10; k++) hp.h[k] = ctx->h[k];
     const uint32_t* perm = nullptr;
