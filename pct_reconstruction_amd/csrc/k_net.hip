@@ -80,125 +80,167 @@ __device__ __forceinline__ uint4 load_in8(const ConvIn& in, int D, int H, int W,
     return r;
 }
 
-// Forward 3x3x3 convolution (also the backward-data pass with flipped weights).
-// A wave computes 16 voxels x 16*NT output channels; a workgroup 64 voxels.
-// Wt: bf16 [Cout][Kp], k = tap * Cin + c; bias may be null.
-template <int NT>
-__global__ void __launch_bounds__(kBlock) k_conv_fwd(ConvIn in, int D, int H, int W, int Kp,
-                                                      const uint16_t* __restrict__ Wt,
-                                                      const float* __restrict__ bias, int relu,
-                                                      uint16_t* __restrict__ out)
+// 3x3x3 convolution (forward, and backward data with flipped weights).  A workgroup takes an output tile of
+// 16 (x) x ty x tz voxels: it loads the tile's input halo (all Cin channels, zeros outside the grid) into LDS once.
+// Its four waves are 4 / wn groups of rows by wn groups of output channels; a wave computes RW rows of 16 voxels x
+// 16 NT channels, so that an input fragment from LDS serves NT matrix products and a weight fragment from the caches
+// RW.  Each output's products are accumulated in the order of k = tap * Cin + c, 32 to an instruction, whatever the
+// tile: the values do not depend on the shape.
+// The weights are the first operand: a lane then holds four consecutive output channels of one voxel.
+// A voxel's channels are padded in LDS to an odd number of 16-byte units, so that the 16 voxels of a fragment lie in
+// different banks.  The LDS offsets of the k groups come from a table (no division in the loop), and the fragments of
+// kSteps k steps are read ahead of their products.
+// Bound by the LDS reads of the input fragments where there are 16 or 32 output channels, by the matrix cores at 48
+// and more.  The seven layers on 128 x 128 x 32: 732 us before (weights fetched row by row for every step, divisions
+// in the loop, 128 workgroups without a halo at 192 channels), 140 now; 48 -> 16 channels on 256 x 256 x 96 1.6 ms,
+// now 0.70 (0.24 at the card's matrix rate), 16 -> 48 0.48.
+constexpr int kTileX = 16, kHaloX = kTileX + 2, kSteps = 4;
+
+struct ConvShape {
+    int ty, tz, wn;
+    int stride;                    // 16-byte units per voxel in LDS
+    int row_units, row_q, row_r;   // 16-byte loads of a halo row, and kBlock split by them
+    uint32_t by_groups, by_hy;     // reciprocals, 16 bits of fraction
+};
+
+// Wt: bf16 [k step of 32][16 output channels][lane][8] (k_pack_weights); bias may be null
+template <int RW, int NT>
+__global__ void __launch_bounds__(kBlock) k_conv(ConvIn in, int D, int H, int W, ConvShape sh,
+                                                 const uint16_t* __restrict__ Wt, const float* __restrict__ bias, int relu,
+                                                 uint16_t* __restrict__ out)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t nvox = (int64_t)D * H * W;
-    const int64_t m0 = ((int64_t)blockIdx.x * 4 + wave) * 16;
-    if (m0 >= nvox) return;  // uniform over the wave
-    const int Cin = in.ca + in.cb, K = 27 * Cin, Cout = 16 * NT;
-    const int g = lane >> 4, i = lane & 15;
-    const int64_t m = m0 + i;
-    const bool mv = m < nvox;
-    const int x = (int)(m % W), y = (int)((m / W) % H), z = (int)(m / ((int64_t)W * H));
-    f32x4 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kc = 0; kc < Kp; kc += 32) {
-        const int k = kc + 8 * g;
-        uint4 av = make_uint4(0, 0, 0, 0);
-        if (mv && k < K) {
-            const int tap = k / Cin, c = k - tap * Cin;
-            av = load_in8(in, D, H, W, z + tap / 9 - 1, y + (tap / 3) % 3 - 1, x + tap % 3 - 1, c);
-        }
-        const bf16x8 a = as_bf16x8(av);
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const bf16x8 b = as_bf16x8(ld16(Wt + (int64_t)(16 * t + i) * Kp + k));
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-        }
+    extern __shared__ uint4 lds[];
+    const int Cin = in.ca + in.cb, groups = Cin / 8, ngroups = 27 * groups, steps = (ngroups + 3) / 4;
+    const int tab_units = (steps * 4 + 4 * kSteps + 3) / 4;  // 16-byte units
+    uint32_t* tab = reinterpret_cast<uint32_t*>(lds);
+    uint4* halo = lds + tab_units;
+    const int HY = sh.ty + 2, HZ = sh.tz + 2;
+    const int tx = blockIdx.x * kTileX, ty = blockIdx.y * sh.ty, tz = blockIdx.z * sh.tz;
+    for (int q = threadIdx.x; q < 4 * tab_units; q += kBlock) {
+        const int tap = q / groups, c = q - tap * groups;
+        tab[q] = q < ngroups ? (uint32_t)(((tap / 9 * HY + tap / 3 % 3) * kHaloX + tap % 3) * sh.stride + c) : 0u;
     }
-    // D[row][col]: lane holds rows 4g..4g+3 of column i
+    {
+        // thread -> 16-byte units t, t + kBlock, ... of the halo, in (row, x, channel group) order
+        const int rows = HY * HZ;
+        int row = (int)threadIdx.x / sh.row_units, rem = (int)threadIdx.x - row * sh.row_units;
+        constexpr int kAhead = 4;
+        while (row < rows) {
+            uint4 v[kAhead];
+            int at[kAhead];
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int co = 16 * t + i;
-        const float bv = bias ? bias[co] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int64_t vox = m0 + 4 * g + r;
-            if (vox < nvox) {
-                float v = acc[t][r] + bv;
-                if (relu) v = v > 0.0f ? v : 0.0f;
-                out[vox * Cout + co] = f2bf(v);
+            for (int u = 0; u < kAhead; u++) {
+                at[u] = -1;
+                if (row < rows) {
+                    const int hx = (int)(((uint32_t)rem * sh.by_groups) >> 16), cg = rem - hx * groups;
+                    const int hz = (int)(((uint32_t)row * sh.by_hy) >> 16), hy = row - hz * HY;
+                    at[u] = (row * kHaloX + hx) * sh.stride + cg;
+                    v[u] = load_in8(in, D, H, W, tz + hz - 1, ty + hy - 1, tx + hx - 1, cg * 8);
+                }
+                row += sh.row_q;
+                rem += sh.row_r;
+                if (rem >= sh.row_units) {
+                    rem -= sh.row_units;
+                    row++;
+                }
             }
+#pragma unroll
+            for (int u = 0; u < kAhead; u++)
+                if (at[u] >= 0) halo[at[u]] = v[u];
         }
-    }
-}
-
-// k_conv_fwd with the input staged in LDS.  A workgroup takes an output tile of 16 (x) x TY (y) x 2 (z)
-// voxels (TY = 4 or 2): it loads the tile's 18 x (TY + 2) x 4 input halo (all Cin channels, zeros
-// outside the grid) once, and each wave computes TY / 2 rows of 16 voxels from LDS, so every input
-// voxel is read from memory about once per tile instead of once per tap.  The k order, and so every
-// output value, is that of k_conv_fwd.  LDS: halo voxels * Cin bf16 (dynamic).
-constexpr int kTileX = 16, kTileZ = 2;
-constexpr int halo_vox(int ty) { return (kTileX + 2) * (ty + 2) * (kTileZ + 2); }
-
-template <int NT, int TY>
-__global__ void __launch_bounds__(kBlock) k_conv_fwd_tiled(ConvIn in, int D, int H, int W, int Kp,
-                                                            const uint16_t* __restrict__ Wt,
-                                                            const float* __restrict__ bias, int relu,
-                                                            uint16_t* __restrict__ out)
-{
-    constexpr int HX = kTileX + 2, HY = TY + 2, NV = halo_vox(TY), RPW = TY * kTileZ / 4;  // rows per wave
-    extern __shared__ uint4 tile4[];
-    const int Cin = in.ca + in.cb, K = 27 * Cin, Cout = 16 * NT;
-    const int tx = blockIdx.x * kTileX, ty = blockIdx.y * TY, tz = blockIdx.z * kTileZ;
-    const int groups = Cin / 8;
-    for (int t = threadIdx.x; t < NV * groups; t += kBlock) {
-        const int v = t / groups, cg = t - v * groups;
-        const int hx = v % HX, hy = (v / HX) % HY, hz = v / (HX * HY);
-        tile4[(v * Cin + cg * 8) / 8] = load_in8(in, D, H, W, tz + hz - 1, ty + hy - 1, tx + hx - 1, cg * 8);
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, i = lane & 15;
-    f32x4 acc[RPW][NT];
+    const int wn = wave % sh.wn, wm = wave / sh.wn;
+    const int ntiles = NT * sh.wn, Cout = 16 * ntiles;
+    const uint4* rows[RW];
+    f32x4 acc[RW][NT];
 #pragma unroll
-    for (int rr = 0; rr < RPW; rr++)
+    for (int rr = 0; rr < RW; rr++) {
+        const int r = RW * wm + rr, rz = r / sh.ty, ry = r - rz * sh.ty;
+        rows[rr] = halo + ((rz * HY + ry) * kHaloX + i) * sh.stride;
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[rr][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kc = 0; kc < Kp; kc += 32) {
-        const int k = kc + 8 * g;
-        const int tap = k / Cin, c = k - tap * Cin;
-        const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;  // offsets + 1
-        bf16x8 b[NT];
+    }
+    const uint4* wp = reinterpret_cast<const uint4*>(Wt) + (int64_t)(NT * wn) * 64 + lane;
+    const int wstep = ntiles * 64;  // 16-byte units of the weights of one step
+    uint32_t off[kSteps];
+    uint4 w[kSteps][NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) b[t] = as_bf16x8(ld16(Wt + (int64_t)(16 * t + i) * Kp + k));
+    for (int u = 0; u < kSteps; u++) {
+        off[u] = tab[4 * u + g];
+        const int s = u < steps ? u : steps - 1;
 #pragma unroll
-        for (int rr = 0; rr < RPW; rr++) {
-            const int r = RPW * wave + rr, ry = r % TY, rz = r / TY;
-            uint4 av = make_uint4(0, 0, 0, 0);
-            if (k < K) av = tile4[((((rz + dz) * HY + (ry + dy)) * HX + (i + dx)) * Cin + c) / 8];
-            const bf16x8 a = as_bf16x8(av);
+        for (int t = 0; t < NT; t++) w[u][t] = wp[(int64_t)s * wstep + t * 64];
+    }
+    const int full = ngroups / 4;  // steps without padding
+    int s0 = 0;
+    for (; s0 + kSteps <= full; s0 += kSteps) {
+        uint4 a[kSteps][RW], wnext[kSteps][NT];
 #pragma unroll
-            for (int t = 0; t < NT; t++) acc[rr][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], acc[rr][t], 0, 0, 0);
+        for (int u = 0; u < kSteps; u++)
+#pragma unroll
+            for (int rr = 0; rr < RW; rr++) a[u][rr] = rows[rr][off[u]];
+#pragma unroll
+        for (int u = 0; u < kSteps; u++) {
+            off[u] = tab[4 * (s0 + kSteps + u) + g];
+            const int s = s0 + kSteps + u < steps ? s0 + kSteps + u : steps - 1;
+#pragma unroll
+            for (int t = 0; t < NT; t++) wnext[u][t] = wp[(int64_t)s * wstep + t * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < kSteps; u++)
+#pragma unroll
+            for (int rr = 0; rr < RW; rr++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    acc[rr][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[u][t]), as_bf16x8(a[u][rr]), acc[rr][t], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < kSteps; u++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) w[u][t] = wnext[u][t];
+    }
+#pragma unroll
+    for (int u = 0; u < kSteps; u++) {
+        if (s0 + u >= steps) break;
+        const bool in_k = 4 * (s0 + u) + g < ngroups;
+#pragma unroll
+        for (int rr = 0; rr < RW; rr++) {
+            uint4 a = rows[rr][off[u]];
+            a.x = in_k ? a.x : 0u;
+            a.y = in_k ? a.y : 0u;
+            a.z = in_k ? a.z : 0u;
+            a.w = in_k ? a.w : 0u;
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                acc[rr][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(w[u][t]), as_bf16x8(a), acc[rr][t], 0, 0, 0);
         }
     }
-    // D[row][col]: lane holds rows 4g..4g+3 (x = tx + 4g + r) of column i
+    // D[row][col]: lane holds channels 4g..4g+3 of voxel i
+    const int x = tx + i;
+    if (x >= W) return;
 #pragma unroll
-    for (int rr = 0; rr < RPW; rr++) {
-        const int rw = RPW * wave + rr, y = ty + rw % TY, z = tz + rw / TY;
-        if (y >= H || z >= D) continue;
+    for (int t = 0; t < NT; t++) {
+        const int co = 16 * (NT * wn + t) + 4 * g;
+        float bv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (bias) {
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const int co = 16 * t + i;
-            const float bv = bias ? bias[co] : 0.0f;
+            for (int r = 0; r < 4; r++) bv[r] = bias[co + r];
+        }
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int x = tx + 4 * g + r;
-                if (x < W) {
-                    float v = acc[rr][t][r] + bv;
-                    if (relu) v = v > 0.0f ? v : 0.0f;
-                    out[(((int64_t)z * H + y) * W + x) * Cout + co] = f2bf(v);
-                }
+        for (int rr = 0; rr < RW; rr++) {
+            const int r = RW * wm + rr, rz = r / sh.ty, y = ty + (r - rz * sh.ty), z = tz + rz;
+            if (y >= H || z >= D) continue;
+            uint32_t e[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                float v = acc[rr][t][q] + bv[q];
+                if (relu) v = v > 0.0f ? v : 0.0f;
+                e[q] = f2bf(v);
             }
+            *reinterpret_cast<uint2*>(out + (((int64_t)z * H + y) * W + x) * Cout + co) =
+                make_uint2(e[0] | e[1] << 16, e[2] | e[3] << 16);
         }
     }
 }
@@ -301,25 +343,36 @@ __global__ void k_reduce_bias(int nchunks, int Cout, const float* __restrict__ p
     grad[co] = s;
 }
 
-// master [Cout][27][Cin] fp32 -> forward bf16 [Cout][Kp] and flipped bf16 [Cin][Kpf] (k' = tap' * Cout + co,
-// tap' = 26 - tap), zero padding beyond K
+// k index and output channel of element idx of a weight array in fragment order: [k step][ntiles][lane][8]
+__device__ __forceinline__ void frag_index(int64_t idx, int ntiles, int* co, int* k)
+{
+    const int j = (int)(idx & 7), lane = (int)(idx >> 3) & 63;
+    const int64_t f = idx >> 9;
+    *co = 16 * (int)(f % ntiles) + (lane & 15);
+    *k = 32 * (int)(f / ntiles) + 8 * (lane >> 4) + j;
+}
+
+// master [Cout][27][Cin] fp32 -> bf16 fragments of the forward weights (k = tap * Cin + c) and of the flipped ones
+// (k' = tap' * Cout + co, tap' = 26 - tap, output channels Cin), zeros beyond K.  An input of 8 channels has no
+// flipped weights: its gradient is not formed.
 __global__ void k_pack_weights(const float* __restrict__ w, int Cin, int Cout, int Kp, int Kpf,
                                uint16_t* __restrict__ wt, uint16_t* __restrict__ wf)
 {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t n1 = (int64_t)Cout * Kp, n2 = (int64_t)Cin * Kpf;
+    const int64_t n1 = (int64_t)Cout * Kp, n2 = Cin % 16 ? 0 : (int64_t)Cin * Kpf;
+    int co, k;
     if (idx < n1) {
-        const int co = (int)(idx / Kp), k = (int)(idx % Kp);
+        frag_index(idx, Cout / 16, &co, &k);
         wt[idx] = k < 27 * Cin ? f2bf(w[(int64_t)co * 27 * Cin + k]) : (uint16_t)0;
     } else if (idx < n1 + n2) {
-        const int64_t j = idx - n1;
-        const int c = (int)(j / Kpf), kf = (int)(j % Kpf);
+        int c;
+        frag_index(idx - n1, Cin / 16, &c, &k);
         uint16_t v = 0;
-        if (kf < 27 * Cout) {
-            const int tapf = kf / Cout, co = kf % Cout;
-            v = f2bf(w[((int64_t)co * 27 + (26 - tapf)) * Cin + c]);
+        if (k < 27 * Cout) {
+            const int tapf = k / Cout, o = k % Cout;
+            v = f2bf(w[((int64_t)o * 27 + (26 - tapf)) * Cin + c]);
         }
-        wf[j] = v;
+        wf[idx - n1] = v;
     }
 }
 
@@ -588,51 +641,88 @@ int pack_weights(pct_net* net)
     return PCT_OK;
 }
 
-int launch_conv(pct_net* net, const ConvIn& in, int level, int Kp, const uint16_t* w, const float* bias, int relu,
-                int cout, uint16_t* out)
+// The tile of a convolution and what its kernel derives from it.
+ConvShape conv_shape(int cin, int wn, int rw, int ty, size_t* lds)
+{
+    ConvShape sh{};
+    sh.ty = ty;
+    sh.tz = rw * (4 / wn) / ty;
+    sh.wn = wn;
+    const int groups = cin / 8;
+    sh.stride = groups | 1;
+    sh.row_units = kHaloX * groups;
+    sh.row_q = kBlock / sh.row_units;
+    sh.row_r = kBlock % sh.row_units;
+    sh.by_groups = 65536u / groups + 1;  // exact for x < row_units (at most 432) and rows of a halo
+    sh.by_hy = 65536u / (ty + 2) + 1;
+    const int steps = (27 * groups + 3) / 4;
+    *lds = 16 * ((size_t)(steps * 4 + 4 * kSteps + 3) / 4 + (size_t)kHaloX * (ty + 2) * (sh.tz + 2) * sh.stride);
+    return sh;
+}
+
+template <int RW, int NT>
+int launch_conv_as(pct_net* net, const ConvIn& in, int level, const ConvShape& sh, size_t lds, const uint16_t* w,
+                   const float* bias, int relu, uint16_t* out)
 {
     const int D = net->D >> level, H = net->H >> level, W = net->W >> level;
-    const int64_t nvox = (int64_t)D * H * W;
-    const unsigned grid = (unsigned)((nvox + 63) / 64);
-    hipStream_t s = net->stream;
-    // the input halo in LDS: 16 x 4 x 2 output tiles, or 16 x 2 x 2 for wider inputs
-    const int cin = in.ca + in.cb;
-    const int ty = (size_t)halo_vox(4) * cin * sizeof(uint16_t) <= 64 * 1024 ? 4
-                   : (size_t)halo_vox(2) * cin * sizeof(uint16_t) <= 64 * 1024 ? 2 : 0;
-    if (ty > 0) {
-        const size_t lds = (size_t)halo_vox(ty) * cin * sizeof(uint16_t);
-        const dim3 tg((W + kTileX - 1) / kTileX, (H + ty - 1) / ty, (D + kTileZ - 1) / kTileZ);
-#define PCT_CONV_T(NT)                                                                                            \
-    if (ty == 4)                                                                                                  \
-        hipLaunchKernelGGL((k_conv_fwd_tiled<NT, 4>), tg, dim3(kBlock), lds, s, in, D, H, W, Kp, w, bias, relu, out); \
-    else                                                                                                          \
-        hipLaunchKernelGGL((k_conv_fwd_tiled<NT, 2>), tg, dim3(kBlock), lds, s, in, D, H, W, Kp, w, bias, relu, out);
-        switch (cout) {
-        case 16: PCT_CONV_T(1) break;
-        case 32: PCT_CONV_T(2) break;
-        case 48: PCT_CONV_T(3) break;
-        case 64: PCT_CONV_T(4) break;
-        case 96: PCT_CONV_T(6) break;
-        case 128: PCT_CONV_T(8) break;
-        case 192: PCT_CONV_T(12) break;
-        default: net->err = "unsupported channel count"; return PCT_E_ARG;
-        }
-#undef PCT_CONV_T
-        NET_HIP(net, hipGetLastError());
-        return PCT_OK;
-    }
-    switch (cout) {
-    case 16: hipLaunchKernelGGL(k_conv_fwd<1>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    case 32: hipLaunchKernelGGL(k_conv_fwd<2>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    case 48: hipLaunchKernelGGL(k_conv_fwd<3>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    case 64: hipLaunchKernelGGL(k_conv_fwd<4>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    case 96: hipLaunchKernelGGL(k_conv_fwd<6>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    case 128: hipLaunchKernelGGL(k_conv_fwd<8>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    case 192: hipLaunchKernelGGL(k_conv_fwd<12>, dim3(grid), dim3(kBlock), 0, s, in, D, H, W, Kp, w, bias, relu, out); break;
-    default: net->err = "unsupported channel count"; return PCT_E_ARG;
-    }
+    const dim3 grid((W + kTileX - 1) / kTileX, (H + sh.ty - 1) / sh.ty, (D + sh.tz - 1) / sh.tz);
+    if (lds > 64 * 1024)
+        NET_HIP(net, hipFuncSetAttribute((const void*)k_conv<RW, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((k_conv<RW, NT>), grid, dim3(kBlock), lds, net->stream, in, D, H, W, sh, w, bias, relu, out);
     NET_HIP(net, hipGetLastError());
     return PCT_OK;
+}
+
+// The tile's rule.  More rows per wave use a weight fragment more often, and fewer waves along the channels an input
+// fragment; both need rows, so fewer workgroups and a larger halo.  In order of rows per wave, and with the channels
+// of 32 and 64 first on fewer waves, the first shape is taken that leaves three workgroups room on a compute unit
+// (54 KB; 64 with the granularity of the shapes) and has 384 of them; a halo of 192 channels needs more than that
+// at any useful size and may take 160 KB.  Measured (us, taken | next): on 256 x 256 x 96, 48 -> 16 channels 8 rows in
+// 47 KB 698 | 16 rows in 71 KB 738; 96 -> 32 at half size 4 rows in 59 KB 293 | 8 in 89 KB 380; 192 -> 64 at a quarter
+// 4 rows in 115 KB 160 | 1 in 65 KB 205; 32 -> 64 there 8 rows, 768 workgroups 18.0 | 4 rows 19.9; on 128 x 128 x 32,
+// 16 -> 32 at half size 8 rows, 512 workgroups 7.7 | 16 rows, 256 workgroups 9.5.
+int launch_conv(pct_net* net, const ConvIn& in, int level, const uint16_t* w, const float* bias, int relu, int cout,
+                uint16_t* out)
+{
+    const int tiles = cout / 16, cin = in.ca + in.cb;
+    const int64_t D = net->D >> level, H = net->H >> level, W = net->W >> level;
+    struct Split {
+        int nt, wn;
+    } split[2];
+    int n_split = 0;
+    for (int wn = 1; wn <= 4; wn *= 2)
+        if (tiles % wn == 0 && tiles / wn <= 3 && n_split < 2) split[n_split++] = Split{tiles / wn, wn};
+    if (cout % 16 || n_split == 0) {
+        net->err = "unsupported channel count";
+        return PCT_E_ARG;
+    }
+    int rw = 1, nt = split[n_split - 1].nt, wn = split[n_split - 1].wn;  // the most workgroups, if none is taken
+    int ty = wn == 4 ? 1 : 2;
+    bool found = false;
+    for (const size_t room : {(size_t)64 << 10, (size_t)160 << 10})
+        for (int r = 4; r >= 1 && !found; r /= 2)
+            for (int k = 0; k < n_split && !found; k++) {
+                const int rows = r * 4 / split[k].wn, t = rows >= 8 ? 4 : rows >= 2 ? 2 : 1;
+                size_t lds = 0;
+                const ConvShape sh = conv_shape(cin, split[k].wn, r, t, &lds);
+                const int64_t groups = (W + kTileX - 1) / kTileX * ((H + t - 1) / t) * ((D + sh.tz - 1) / sh.tz);
+                if (lds > room || groups < 384) continue;
+                rw = r;
+                ty = t;
+                nt = split[k].nt;
+                wn = split[k].wn;
+                found = true;
+            }
+    size_t lds = 0;
+    const ConvShape sh = conv_shape(cin, wn, rw, ty, &lds);
+#define PCT_CONV(RW, NT) \
+    if (rw == RW && nt == NT) return launch_conv_as<RW, NT>(net, in, level, sh, lds, w, bias, relu, out);
+    PCT_CONV(4, 1) PCT_CONV(4, 2) PCT_CONV(4, 3)
+    PCT_CONV(2, 1) PCT_CONV(2, 2) PCT_CONV(2, 3)
+    PCT_CONV(1, 1) PCT_CONV(1, 2) PCT_CONV(1, 3)
+#undef PCT_CONV
+    net->err = "unsupported channel count";
+    return PCT_E_ARG;
 }
 
 constexpr int64_t kBiasChunk = 256;  // voxels per bias-gradient partial
@@ -718,7 +808,7 @@ int net_forward(pct_net* net, const float* fbp, const uint8_t* hull, const float
     const int level[kLayers] = {0, 1, 2, 3, 2, 1, 0};
     for (int l = 0; l < kLayers; l++) {
         auto& Ly = net->L[l];
-        PCT_TRY(launch_conv(net, conv_input(net, l), level[l], Ly.Kp, Ly.wt, net->p + Ly.b_off, 1, Ly.cout, outs[l]));
+        PCT_TRY(launch_conv(net, conv_input(net, l), level[l], Ly.wt, net->p + Ly.b_off, 1, Ly.cout, outs[l]));
         if (l < 3) {
             const int D = net->D >> l, H = net->H >> l, W = net->W >> l;
             const int64_t n = (int64_t)(D / 2) * (H / 2) * (W / 2) * Ly.cout;
@@ -776,7 +866,7 @@ int net_backward(pct_net* net, const uint8_t* hull, const float* target)
         PCT_TRY(launch_wgrad(net, in, level, l, net->g_dd[d]));
         // concat gradient: conv of dPre with flipped weights (Cin' = Cout, Cout' = Cin)
         ConvIn gin{net->g_dd[d], nullptr, Ly.cout, 0, 0};
-        PCT_TRY(launch_conv(net, gin, level, Ly.Kpf, Ly.wf, nullptr, 0, Ly.cin, net->g_cat[d]));
+        PCT_TRY(launch_conv(net, gin, level, Ly.wf, nullptr, 0, Ly.cin, net->g_cat[d]));
         const int D = net->D >> level, H = net->H >> level, W = net->W >> level;
         const int ca = in.ca;
         // coarse part -> dPre of the tensor one level down (dec2, dec3 or enc4)
@@ -804,7 +894,7 @@ int net_backward(pct_net* net, const uint8_t* hull, const float* target)
         if (l > 0) {
             // gradient of the pooled input of this layer
             ConvIn gin{net->g_e[l], nullptr, Ly.cout, 0, 0};
-            PCT_TRY(launch_conv(net, gin, level, Ly.Kpf, Ly.wf, nullptr, 0, Ly.cin, net->g_pool[l - 1]));
+            PCT_TRY(launch_conv(net, gin, level, Ly.wf, nullptr, 0, Ly.cin, net->g_pool[l - 1]));
         }
     }
     NET_HIP(net, hipGetLastError());
