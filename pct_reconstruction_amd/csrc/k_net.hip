@@ -27,6 +27,7 @@
 // voxel chunks into FP32 partials that a second kernel sums in chunk order (deterministic).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -245,102 +246,138 @@ __global__ void __launch_bounds__(kBlock) k_conv(ConvIn in, int D, int H, int W,
     }
 }
 
-// Weight gradient partials: partial[chunk][co][k] = sum over the chunk's voxels v of
-// A[v][k] * G[v][co], A the convolution input gathered as in the forward pass, G = dL/d(pre-ReLU).
-// Workgroup: one 64-wide k tile (16 k per wave) x all Cout, over vchunk voxels in slices of 32.
-template <int NT>
-__global__ void __launch_bounds__(kBlock) k_conv_wgrad(ConvIn in, int D, int H, int W, int Kp,
-                                                        const uint16_t* __restrict__ G, int vchunk,
-                                                        float* __restrict__ partial)
+// Weight gradient partials: partial[chunk][co][k] = sum over the chunk's voxels v of A[v][k] * G[v][co], A the
+// convolution input gathered as in the forward pass, G = dL/d(pre-ReLU); entry k = K is the sum of G[v][co], the bias
+// gradient.  The contraction runs over voxels, so a lane's eight elements are eight voxels of one channel: a tile of
+// 16 x kGY x kGZ voxels is transposed into LDS, channel by channel, rows along x.  A workgroup takes 16 input channels
+// (blockIdx.y) and 16 NT output channels (blockIdx.z) over a chunk of tiles (blockIdx.x); its three waves take the taps'
+// three dz.  An input row read once serves its three dx: dx = 0 and 2 are whole registers of it, dx = 1 a shift by 16
+// bits.  Channels lie an odd number of 16-byte units apart, so that the fragment reads are free of bank conflicts.
+// Bound by the staging (two 16-byte loads and eight 4-byte LDS writes for each 16 elements) at 16 and 32 output
+// channels.  On 128 x 128 x 32 the seven layers take 275 us; one 64-wide slice of k per workgroup, staged element by
+// element for one product per wave and barrier, took 1680, and the bias gradients apart another 1730.
+constexpr int kGY = 8, kGZ = 2, kGRows = kGY * kGZ, kGBlock = 192;
+constexpr int kGHalo = (kGY + 2) * (kGZ + 2);
+constexpr int kGInStride = kGHalo * 12 + 4, kGOutStride = kGRows * 8 + 4;  // 4-byte words per channel
+static_assert((kGInStride / 4) % 2 == 1 && (kGOutStride / 4) % 2 == 1, "channels in different banks");
+
+// 8 channels of two voxels into rows of 8 channels, 4 bytes each
+__device__ __forceinline__ void put_pair(uint32_t* at, int stride, uint4 a, uint4 b)
 {
-    constexpr int Cout = 16 * NT;
-    __shared__ __align__(16) uint16_t As[64][40];      // [k][v], rows padded to 80 B
-    __shared__ __align__(16) uint16_t Bs[Cout][40];    // [co][v]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, i = lane & 15;
-    const int64_t nvox = (int64_t)D * H * W;
-    const int Cin = in.ca + in.cb, K = 27 * Cin;
-    const int kt = blockIdx.x * 64;
-    const int64_t v_begin = (int64_t)blockIdx.y * vchunk;
-    int64_t v_end = v_begin + vchunk;
-    if (v_end > nvox) v_end = nvox;
-    f32x4 acc[NT];
+    const uint32_t va[4] = {a.x, a.y, a.z, a.w}, vb[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // staging roles: A: thread -> (voxel tid/8, k group tid%8); B: thread -> (voxel tid%32, co group tid/32)
-    const int av = tid >> 3, ak = kt + 8 * (tid & 7);
-    for (int64_t v0 = v_begin; v0 < v_end; v0 += 32) {
-        {
-            const int64_t v = v0 + av;
-            uint4 a = make_uint4(0, 0, 0, 0);
-            if (v < v_end && ak < K) {
-                const int x = (int)(v % W), y = (int)((v / W) % H), z = (int)(v / ((int64_t)W * H));
-                const int tap = ak / Cin, c = ak - tap * Cin;
-                a = load_in8(in, D, H, W, z + tap / 9 - 1, y + (tap / 3) % 3 - 1, x + tap % 3 - 1, c);
-            }
-            const uint16_t* e = reinterpret_cast<const uint16_t*>(&a);
-            const int kl = 8 * (tid & 7);
-#pragma unroll
-            for (int j = 0; j < 8; j++) As[kl + j][av] = e[j];
-        }
-        for (int q = tid; q < 32 * (Cout / 8); q += kBlock) {
-            const int bv = q & 31, cg = (q >> 5) * 8;
-            const int64_t v = v0 + bv;
-            uint4 b = make_uint4(0, 0, 0, 0);
-            if (v < v_end) b = ld16(G + v * Cout + cg);
-            const uint16_t* e = reinterpret_cast<const uint16_t*>(&b);
-#pragma unroll
-            for (int j = 0; j < 8; j++) Bs[cg + j][bv] = e[j];
-        }
-        __syncthreads();
-        const bf16x8 a = as_bf16x8(*reinterpret_cast<const uint4*>(&As[16 * wave + i][8 * g]));
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const bf16x8 b = as_bf16x8(*reinterpret_cast<const uint4*>(&Bs[16 * t + i][8 * g]));
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-        }
-        __syncthreads();
+    for (int j = 0; j < 4; j++) {
+        at[(2 * j) * stride] = (va[j] & 0xffffu) | vb[j] << 16;
+        at[(2 * j + 1) * stride] = va[j] >> 16 | (vb[j] & 0xffff0000u);
     }
-    // D[k][co]: lane holds k rows 4g..4g+3 (within the wave's 16) of column co = 16t + i
-    float* P = partial + (int64_t)blockIdx.y * Cout * Kp;
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) P[(int64_t)(16 * t + i) * Kp + kt + 16 * wave + 4 * g + r] = acc[t][r];
 }
 
-// grad[co][k] (k < K) = sum over chunks of partial[chunk][co][k], in chunk order
-__global__ void k_reduce_partials(int nchunks, int Cout, int K, int Kp, const float* __restrict__ partial,
+template <int NT>
+__global__ void __launch_bounds__(kGBlock) k_conv_wgrad(ConvIn in, int D, int H, int W, const uint16_t* __restrict__ G,
+                                                        int Cout, int tiles_x, int tiles_y, int tiles, int per_chunk,
+                                                        float* __restrict__ partial)
+{
+    __shared__ __align__(16) uint32_t As[16 * kGInStride];
+    __shared__ __align__(16) uint32_t Gs[16 * NT * kGOutStride];
+    const int Cin = in.ca + in.cb, K = 27 * Cin, Kq = K + 4;
+    const int c0 = 16 * blockIdx.y, co0 = 16 * NT * blockIdx.z, cgs = min(Cin - c0, 16) / 8;
+    const int lane = threadIdx.x & 63, dz = threadIdx.x >> 6, g = lane >> 4, i = lane & 15;
+    const int ic = cgs == 1 ? i & 7 : i;  // the rows of 8 missing channels are not written
+    const bool bias = dz == 0 && blockIdx.y == 0;
+    const bf16x8 ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+    f32x4 acc[3][3][NT], accb[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        accb[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 9; q++) acc[q / 3][q % 3][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int t0 = blockIdx.x * per_chunk, t1 = min(t0 + per_chunk, tiles);
+    for (int tile = t0; tile < t1; tile++) {
+        const int tx = tile % tiles_x * 16, ty = tile / tiles_x % tiles_y * kGY, tz = tile / (tiles_x * tiles_y) * kGZ;
+        __syncthreads();
+        for (int q = threadIdx.x; q < cgs * kGHalo * 9; q += kGBlock) {
+            const int cg = q / (kGHalo * 9), r = q - cg * (kGHalo * 9), row = r / 9, p = r - row * 9;
+            const int z = tz + row / (kGY + 2) - 1, y = ty + row % (kGY + 2) - 1, x = tx + 2 * p - 1, c = c0 + 8 * cg;
+            const uint4 a = load_in8(in, D, H, W, z, y, x, c), b = load_in8(in, D, H, W, z, y, x + 1, c);
+            put_pair(As + 8 * cg * kGInStride + row * 12 + p, kGInStride, a, b);
+        }
+        for (int q = threadIdx.x; q < 2 * NT * kGRows * 8; q += kGBlock) {
+            const int cg = q / (kGRows * 8), row = q / 8 % kGRows, p = q & 7;
+            const int z = tz + row / kGY, y = ty + row % kGY, x = tx + 2 * p;
+            uint4 a = make_uint4(0, 0, 0, 0), b = a;
+            if (z < D && y < H) {
+                const uint16_t* src = G + (((int64_t)z * H + y) * W + x) * Cout + co0 + 8 * cg;
+                if (x < W) a = ld16(src);
+                if (x + 1 < W) b = ld16(src + Cout);
+            }
+            put_pair(Gs + 8 * cg * kGOutStride + row * 8 + p, kGOutStride, a, b);
+        }
+        __syncthreads();
+#pragma unroll 2
+        for (int s = 0; s < kGRows / 2; s++) {
+            // the contraction's 32 voxels: two rows of 16, a lane's eight in row r from x = 8 (g & 1) on
+            const int r = 2 * s + (g >> 1), ry = r % kGY, rz = r / kGY;
+            bf16x8 b[NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                b[t] = as_bf16x8(*reinterpret_cast<const uint4*>(Gs + (16 * t + i) * kGOutStride + r * 8 + 4 * (g & 1)));
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                const uint32_t* src = As + ic * kGInStride + ((rz + dz) * (kGY + 2) + ry + dy) * 12 + 4 * (g & 1);
+                const uint4 d = *reinterpret_cast<const uint4*>(src);
+                const uint32_t e = src[4];
+                const uint4 a1 = make_uint4(__builtin_amdgcn_alignbit(d.y, d.x, 16), __builtin_amdgcn_alignbit(d.z, d.y, 16),
+                                            __builtin_amdgcn_alignbit(d.w, d.z, 16), __builtin_amdgcn_alignbit(e, d.w, 16));
+                const uint4 a2 = make_uint4(d.y, d.z, d.w, e);
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    acc[dy][0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(d), b[t], acc[dy][0][t], 0, 0, 0);
+                    acc[dy][1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1), b[t], acc[dy][1][t], 0, 0, 0);
+                    acc[dy][2][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a2), b[t], acc[dy][2][t], 0, 0, 0);
+                }
+            }
+            if (bias) {
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    accb[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[t], accb[t], 0, 0, 0);
+            }
+        }
+    }
+    // D[c][co]: lane holds channels 4g..4g+3 of column co
+    float* P = partial + (int64_t)blockIdx.x * Cout * Kq;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        float* row = P + (int64_t)(co0 + 16 * t + i) * Kq;
+        if (8 * cgs > 4 * g) {
+#pragma unroll
+            for (int q = 0; q < 9; q++)
+                *reinterpret_cast<f32x4*>(row + (9 * dz + q) * Cin + c0 + 4 * g) = acc[q / 3][q % 3][t];
+        }
+        if (bias && g == 0) row[K] = accb[t][0];
+    }
+}
+
+// grad[co][k] (k < K), then the bias gradients: sums over chunks of partial[chunk][co][k], in chunk order
+__global__ void k_reduce_partials(int nchunks, int Cout, int K, const float* __restrict__ partial,
                                   float* __restrict__ grad)
 {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)Cout * K) return;
-    const int co = (int)(idx / K), k = (int)(idx % K);
+    if (idx >= (int64_t)Cout * (K + 1)) return;
+    const int co = (int)(idx / (K + 1)), k = (int)(idx % (K + 1)), Kq = K + 4;
+    const float* p = partial + (int64_t)co * Kq + k;
+    const int64_t step = (int64_t)Cout * Kq;
     float s = 0.0f;
-    for (int c = 0; c < nchunks; c++) s += partial[((int64_t)c * Cout + co) * Kp + k];
-    grad[idx] = s;
-}
-
-// bias gradient partials: partial[chunk][co] = sum of G[v][co] over the chunk's voxels
-__global__ void k_bias_partials(int64_t nvox, int Cout, int vchunk, const uint16_t* __restrict__ G,
-                                float* __restrict__ partial)
-{
-    const int co = threadIdx.x;
-    if (co >= Cout) return;
-    const int64_t v0 = (int64_t)blockIdx.x * vchunk;
-    int64_t v1 = v0 + vchunk;
-    if (v1 > nvox) v1 = nvox;
-    float s = 0.0f;
-    for (int64_t v = v0; v < v1; v++) s += bf2f(G[v * Cout + co]);
-    partial[(int64_t)blockIdx.x * Cout + co] = s;
-}
-__global__ void k_reduce_bias(int nchunks, int Cout, const float* __restrict__ partial, float* __restrict__ grad)
-{
-    const int co = threadIdx.x;
-    if (co >= Cout) return;
-    float s = 0.0f;
-    for (int c = 0; c < nchunks; c++) s += partial[(int64_t)c * Cout + co];
-    grad[co] = s;
+    int c = 0;
+    for (; c + 8 <= nchunks; c += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = p[(c + u) * step];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; c < nchunks; c++) s += p[c * step];
+    grad[k < K ? (int64_t)co * K + k : (int64_t)Cout * K + co] = s;
 }
 
 // k index and output channel of element idx of a weight array in fragment order: [k step][ntiles][lane][8]
@@ -525,13 +562,20 @@ __global__ void k_head_bwd(int64_t nvox, double inv_n, const uint16_t* __restric
     }
     if (threadIdx.x < 17) part[(int64_t)blockIdx.x * 17 + threadIdx.x] = s[threadIdx.x][0];
 }
-__global__ void k_reduce_cols(int nrows, int ncols, const float* __restrict__ part, float* __restrict__ out)
+// out[c] = sum over rows of part[row][c]; one workgroup per column (one lane per column took 577 us for 2048 rows)
+__global__ void __launch_bounds__(kBlock) k_reduce_cols(int nrows, int ncols, const float* __restrict__ part,
+                                                        float* __restrict__ out)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncols) return;
-    float s = 0.0f;
-    for (int r = 0; r < nrows; r++) s += part[(int64_t)r * ncols + c];
-    out[c] = s;
+    __shared__ float s[kBlock];
+    float v = 0.0f;
+    for (int r = threadIdx.x; r < nrows; r += kBlock) v += part[(int64_t)r * ncols + blockIdx.x];
+    s[threadIdx.x] = v;
+    __syncthreads();
+    for (int o = kBlock / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
 __global__ void k_adam(int64_t n, float lr, float b1, float b2, float eps, float c1, float c2,
@@ -725,60 +769,48 @@ int launch_conv(pct_net* net, const ConvIn& in, int level, const uint16_t* w, co
     return PCT_E_ARG;
 }
 
-constexpr int64_t kBiasChunk = 256;  // voxels per bias-gradient partial
-
-// split of a weight-gradient launch: about 1024 workgroups of (64-wide k tile, voxel chunk)
-void wgrad_shape(int64_t nvox, int Kp, int64_t* nchunks, int64_t* vchunk)
-{
-    const int ktiles = Kp / 64;
-    int64_t nc = 1024 / ktiles;
-    if (nc < 1) nc = 1;
-    int64_t vc = (nvox + nc - 1) / nc;
-    vc = (vc + 31) / 32 * 32;
-    *vchunk = vc;
-    *nchunks = (nvox + vc - 1) / vc;
-}
-
-// floats of partial sums the weight and bias gradients of layer l need
-int64_t partial_need(const pct_net* net, int l)
+// Split of a weight-gradient launch: about 768 workgroups (three of them fill a compute unit's matrix cores and hide
+// each other's staging), with at most 32 MB of partial sums.
+struct WgradShape {
+    int nt, ctiles, groups, tiles_x, tiles_y, tiles, per_chunk, chunks;
+    int64_t chunk_floats;
+};
+WgradShape wgrad_shape(const pct_net* net, int l)
 {
     const auto& Ly = net->L[l];
-    const int64_t nvox = net->nv[Ly.level];
-    int64_t nc = 0, vc = 0;
-    wgrad_shape(nvox, Ly.Kp, &nc, &vc);
-    const int64_t a = nc * Ly.cout * Ly.Kp, b = (nvox + kBiasChunk - 1) / kBiasChunk * Ly.cout;
-    return a > b ? a : b;
+    const int D = net->D >> Ly.level, H = net->H >> Ly.level, W = net->W >> Ly.level;
+    WgradShape w{};
+    w.nt = Ly.cout % 64 == 0 ? 4 : Ly.cout % 32 == 0 ? 2 : 1;
+    w.ctiles = (Ly.cin + 15) / 16;
+    w.groups = Ly.cout / (16 * w.nt);
+    w.tiles_x = (W + 15) / 16;
+    w.tiles_y = (H + kGY - 1) / kGY;
+    w.tiles = w.tiles_x * w.tiles_y * ((D + kGZ - 1) / kGZ);
+    w.chunk_floats = (int64_t)Ly.cout * (27 * Ly.cin + 4);
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(768 / (w.ctiles * w.groups), (8 << 20) / w.chunk_floats));
+    w.per_chunk = (int)((w.tiles + most - 1) / most);
+    w.chunks = (w.tiles + w.per_chunk - 1) / w.per_chunk;
+    return w;
 }
 
 int launch_wgrad(pct_net* net, const ConvIn& in, int level, int l, const uint16_t* G)
 {
     auto& Ly = net->L[l];
     const int D = net->D >> level, H = net->H >> level, W = net->W >> level;
-    const int64_t nvox = (int64_t)D * H * W;
-    const int ktiles = Ly.Kp / 64;
-    int64_t nchunks = 0, vchunk = 0;
-    wgrad_shape(nvox, Ly.Kp, &nchunks, &vchunk);
-    if (partial_need(net, l) > net->partial_n) {
+    const WgradShape w = wgrad_shape(net, l);
+    if (w.chunks * w.chunk_floats > net->partial_n) {
         net->err = "gradient scratch too small";
         return PCT_E_LIMIT;
     }
     hipStream_t s = net->stream;
-    dim3 grid((unsigned)ktiles, (unsigned)nchunks);
-    switch (Ly.cout) {
-    case 16: hipLaunchKernelGGL(k_conv_wgrad<1>, grid, dim3(kBlock), 0, s, in, D, H, W, Ly.Kp, G, (int)vchunk, net->partial); break;
-    case 32: hipLaunchKernelGGL(k_conv_wgrad<2>, grid, dim3(kBlock), 0, s, in, D, H, W, Ly.Kp, G, (int)vchunk, net->partial); break;
-    case 64: hipLaunchKernelGGL(k_conv_wgrad<4>, grid, dim3(kBlock), 0, s, in, D, H, W, Ly.Kp, G, (int)vchunk, net->partial); break;
-    case 128: hipLaunchKernelGGL(k_conv_wgrad<8>, grid, dim3(kBlock), 0, s, in, D, H, W, Ly.Kp, G, (int)vchunk, net->partial); break;
-    default: net->err = "unsupported channel count"; return PCT_E_ARG;
-    }
-    const int K = 27 * Ly.cin;
-    hipLaunchKernelGGL(k_reduce_partials, dim3(blocks_for((int64_t)Ly.cout * K)), dim3(kBlock), 0, s, (int)nchunks,
-                       Ly.cout, K, Ly.Kp, net->partial, net->g + Ly.w_off);
-    // bias
-    const int64_t nb = (nvox + kBiasChunk - 1) / kBiasChunk;
-    hipLaunchKernelGGL(k_bias_partials, dim3((unsigned)nb), dim3(128), 0, s, nvox, Ly.cout, (int)kBiasChunk, G,
+    const dim3 grid((unsigned)w.chunks, (unsigned)w.ctiles, (unsigned)w.groups);
+    auto kern = w.nt == 4 ? k_conv_wgrad<4> : w.nt == 2 ? k_conv_wgrad<2> : k_conv_wgrad<1>;
+    hipLaunchKernelGGL(kern, grid, dim3(kGBlock), 0, s, in, D, H, W, G, Ly.cout, w.tiles_x, w.tiles_y, w.tiles, w.per_chunk,
                        net->partial);
-    hipLaunchKernelGGL(k_reduce_bias, dim3(1), dim3(128), 0, s, (int)nb, Ly.cout, net->partial, net->g + Ly.b_off);
+    const int K = 27 * Ly.cin;
+    // the bias gradients follow the weights' (b_off = w_off + cout * K)
+    hipLaunchKernelGGL(k_reduce_partials, dim3(blocks_for((int64_t)Ly.cout * (K + 1))), dim3(kBlock), 0, s, w.chunks,
+                       Ly.cout, K, net->partial, net->g + Ly.w_off);
     NET_HIP(net, hipGetLastError());
     return PCT_OK;
 }
@@ -857,7 +889,7 @@ int net_backward(pct_net* net, const uint8_t* hull, const float* target)
     const unsigned nb = blocks_for(n0);
     hipLaunchKernelGGL(k_head_bwd, dim3(nb), dim3(kBlock), 0, s, n0, inv_n, net->dd[0], net->p + net->head_off, hull,
                        net->x0, target, net->g_dd[0], net->head_part);
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(64), 0, s, (int)nb, 17, net->head_part, net->g + net->head_off);
+    hipLaunchKernelGGL(k_reduce_cols, dim3(17), dim3(kBlock), 0, s, (int)nb, 17, net->head_part, net->g + net->head_off);
     // decoder: l = 6 (dec1, level 0), 5 (dec2, level 1), 4 (dec3, level 2)
     for (int d = 0; d < 3; d++) {
         const int l = 6 - d, level = d;
@@ -980,7 +1012,8 @@ int pct_net_create(int columns, int rows, int slices, uint64_t seed, int device,
         (rc = net_alloc(net, &net->head_part, 17 * (int64_t)blocks_for(nv[0]))))
         return fail(rc);
     for (int l = 0; l < kLayers; l++) {
-        const int64_t need = partial_need(net, l);
+        const WgradShape w = wgrad_shape(net, l);
+        const int64_t need = w.chunks * w.chunk_floats;
         net->partial_n = need > net->partial_n ? need : net->partial_n;
     }
     if ((rc = net_alloc(net, &net->partial, net->partial_n))) return fail(rc);
