@@ -186,3 +186,16 @@ def test_tiles_on_imported_lists_with_repeated_voxels(monkeypatch, tmp_path):
             out.append((r.image("x"), r.residual()))
     assert np.array_equal(out[0][0], out[1][0])
     assert abs(out[0][1] - out[1][1]) <= 1e-12 * out[0][1]
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(columns=150, rows=150, slice_thickness=0.5)])
+@pytest.mark.parametrize("every", [37, 2500])
+def test_some_rows_round_in_tiles(monkeypatch, kw, every):
+    """Tiles with a few tiny values: their segments bound their own values, the rows through a tiny one are summed in
+    list order by a whole wavefront (also past 256 entries), the others as they are; bit for bit the sorted lists."""
+    P, data = small_head(n=30000, seed=19, drop_block_size=6000, histories_per_block=640, **kw)
+    rng = np.random.default_rng(4)
+    x = (1.0 + 0.3 * rng.standard_normal(P.num_voxels)).astype(np.float32)
+    x[::every] *= np.float32(1e-12)
+    b = _compare(monkeypatch, P, data, 3, x=x)
+    assert b["prof"]["summed"] > 0
