@@ -297,7 +297,7 @@ struct pct_ctx {
 
     // DROP plan (transposed lists) and the scratch of the atomic DROP kernels
     DropPlan plan;
-    int drop_row_lanes = 16;   // lanes per history in the row kernel (PCT_DROP_ROW_LANES: 4..64)
+    int drop_row_lanes = 0;    // lanes per history in the row kernel: 0 by rule, or 4..64 (PCT_DROP_ROW_LANES)
     int drop_col_voxels = 1;   // voxels per lane in the column kernel (PCT_DROP_COL_VOXELS: 1, 2, 4, 8)
     int drop_flags = PCT_DROP_SPATIAL_ORDER | PCT_DROP_BRICKS | PCT_DROP_COLS_SLICED;  // PCT_DROP_FLAGS
     int mlp_blocks_per_cu = -1;  // MLP list kernel grid: workgroups per CU, 0 = one lane per history, -1 = auto (PCT_MLP_BLOCKS_PER_CU)

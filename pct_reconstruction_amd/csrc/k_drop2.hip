@@ -1396,6 +1396,16 @@ int pct_drop_iterate_plan(pct_ctx* ctx, int iterations, DropTiming* timing)
     return PCT_OK;
 }
 
+// Lanes per history of a block's row kernel, unless the caller set them.  16 lanes with kUnroll loads each read 128
+// entries at a time, and a block of few histories is bound by the latency of each such round: longer lists take 32
+// lanes there (cylinder-2M, 137 entries, DROP of 6 iterations with 16 | 32: blocks of 1600 histories 44.3 | 38.5 ms,
+// 6400 14.3 | 13.4, 12800 9.2 | 9.0).  Blocks that fill the chip are bound by their gathers (head, 227 entries,
+// blocks of 16000: 37.2 | 38.5), and lists of 54 entries have one round with 16 (1.29 | 1.32).
+static int row_lanes(int64_t histories, int64_t entries)
+{
+    return histories <= 8192 && entries > 128 * histories ? 32 : 16;
+}
+
 static int iterate_once(pct_ctx* ctx, DropTiming* timing)
 {
     const pct_params& P = ctx->P;
@@ -1404,13 +1414,14 @@ static int iterate_once(pct_ctx* ctx, DropTiming* timing)
     std::vector<hipEvent_t> ev_rows, ev_cols;
     std::vector<hipEvent_t>* er = timing ? &ev_rows : nullptr;
     std::vector<hipEvent_t>* ec = timing ? &ev_cols : nullptr;
-    const int G = ctx->drop_row_lanes, V = ctx->drop_col_voxels;
+    const int V = ctx->drop_col_voxels;
     const bool xcd = (D.flags & PCT_DROP_XCD_SLABS) != 0;
     const bool bricks = (D.flags & PCT_DROP_BRICKS) != 0;
     const uint32_t* lv = bricks ? D.vox_b : ctx->list_vox;
     float* xx = bricks ? D.x_b : ctx->x;
     for (size_t bi = 0; bi < D.blocks.size(); bi++) {
         const DropPlan::Block& bk = D.blocks[bi];
+        const int G = ctx->drop_row_lanes ? ctx->drop_row_lanes : row_lanes(bk.proc, bk.entries);
         const int64_t hpw = kBlock / G;  // histories per workgroup
         uint32_t rper = 0;
         const dim3 rg(slab_grid((bk.proc + hpw - 1) / hpw, xcd, &rper)), blk(kBlock);
