@@ -15,6 +15,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "internal.h"
+#include "walk.h"
 
 namespace {
 
@@ -44,92 +45,83 @@ __device__ int find_endpoint(const DevGeom& g, const uint32_t* __restrict__ hull
                              int* vxo, int* vyo, int* vzo, int entering)
 {
     const int C = g.C, R = g.R, S = g.S;
-    double x = x_start, y = y_start, z = z_start;
     if (!entering) xy_angle += g.PI;
     const double cxy = cos(xy_angle), sxy = sin(xy_angle), sxz = sin(xz_angle);
-    int x_move = (cxy >= 0) - (cxy <= 0);
-    int y_move = (sxy >= 0) - (sxy <= 0);
-    int z_move = (sxz >= 0) - (sxz <= 0);
-    if (x_move < 0) z_move *= -1;
-    int vx = pct_calc_voxel(g.X0, x, g.VW), vy = pct_calc_voxel(g.Y0, y, g.VH), vz = pct_calc_voxel(g.Z0, z, g.VT);
-    double x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-    double y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-    double z_to_go = pct_dist(g.Z0, z, PCT_Z_INC, z_move, g.VT, vz);
-    int64_t voxel = vx + ((int64_t)vy + (int64_t)vz * R) * C;
+    Walk3 w;
+    w.xs = x_start;
+    w.ys = y_start;
+    w.zs = z_start;
+    w.xm = (cxy >= 0) - (cxy <= 0);
+    w.ym = (sxy >= 0) - (sxy <= 0);
+    w.zm = (sxz >= 0) - (sxz <= 0);
+    if (w.xm < 0) w.zm *= -1;
+    w.vx = pct_calc_voxel(g.X0, x_start, g.VW);
+    w.vy = pct_calc_voxel(g.Y0, y_start, g.VH);
+    w.vz = pct_calc_voxel(g.Z0, z_start, g.VT);
     const double txy = tan(xy_angle), txz = tan(xz_angle);
-    double delta_yx = fabs(txy);
-    double delta_zx = fabs(txz);
-    double delta_zy = fabs(txz / txy);
-    double dy_dx = txy;
-    double dz_dx = txz;
-    double dz_dy = txz / txy;
-    double dx_dy = (double)pct_recipf(txy);
-    double dx_dz = (double)pct_recipf(txz);
-    double dy_dz = (double)pct_tanf(xy_angle) / txz;
-    int hit = 0;
-    bool outside = (vx >= C) || (vy >= R) || (vz >= S) || (vx < 0) || (vy < 0) || (vz < 0);
-    if (!outside) hit = hull_bit(hull, voxel);
-    bool end_walk = outside || hit;
+    w.dy_dx = txy;
+    w.dz_dx = txz;
+    w.dz_dy = txz / txy;
+    w.dx_dy = (double)pct_recipf(txy);
+    w.dx_dz = (double)pct_recipf(txz);
+    w.dy_dz = (double)pct_tanf(xy_angle) / txz;
+    w.ax = w.ay = w.az = w.at = 0;
+    auto outside = [&] {
+        return (uint32_t)w.vx >= (uint32_t)C || (uint32_t)w.vy >= (uint32_t)R || (uint32_t)w.vz >= (uint32_t)S;
+    };
+    auto in_hull = [&]() -> int {
+        return hull_bit(hull, w.vx + ((int64_t)w.vy + (int64_t)w.vz * R) * C);
+    };
     const int cap = 4 * (C + R + S) + 16;
-    int steps = 0;
-    while (!end_walk) {
-        if (z_move != 0) {
-            double x_ext = delta_zx * x_to_go;
-            double y_ext = delta_zy * y_to_go;
-            if ((z_to_go <= x_ext) && (z_to_go <= y_ext)) {
-                vz -= z_move;
-                z = pct_edge(g.Z0, vz, g.VT, PCT_Z_INC, z_move);
-                x = pct_corr(dx_dz, z, z_start, x_start);
-                y = pct_corr(dy_dz, z, z_start, y_start);
-                x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-                z_to_go = g.VT;
-            } else if (x_ext <= y_ext) {
-                vx += x_move;
-                x = pct_edge(g.X0, vx, g.VW, PCT_X_INC, x_move);
-                y = pct_corr(dy_dx, x, x_start, y_start);
-                z = pct_corr(dz_dx, x, x_start, z_start);
-                x_to_go = g.VW;
-                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-                z_to_go = pct_dist(g.Z0, z, PCT_Z_INC, z_move, g.VT, vz);
-            } else {
-                vy -= y_move;
-                y = pct_edge(g.Y0, vy, g.VH, PCT_Y_INC, y_move);
-                x = pct_corr(dx_dy, y, y_start, x_start);
-                z = pct_corr(dz_dy, y, y_start, z_start);
-                x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-                y_to_go = g.VH;
-                z_to_go = pct_dist(g.Z0, z, PCT_Z_INC, z_move, g.VT, vz);
+    int hit = 0, steps = 0;
+    bool end_walk = outside();
+    if (!end_walk) hit = in_hull();
+    end_walk = end_walk || hit;
+    double x = x_start, y = y_start, z = z_start;
+    if (w.zm != 0) {
+        int axis = 3;
+        w.begin(g);
+        while (!end_walk) {
+            int full;
+            bool clamped;
+            axis = w.step(g, &full, &clamped);
+            end_walk = outside();
+            if (!end_walk) hit = in_hull();
+            end_walk = end_walk || hit;
+            if (++steps > cap) {
+                hit = 0;
+                end_walk = true;
             }
-            if (x_to_go == 0) { x_to_go = g.VW; vx += x_move; }
-            if (y_to_go == 0) { y_to_go = g.VH; vy -= y_move; }
-            if (z_to_go == 0) { z_to_go = g.VT; vz -= z_move; }
-            vz = vz > 0 ? vz : 0;
-        } else {
-            double y_ext = y_to_go / delta_yx;
-            if (x_to_go <= y_ext) {
-                vx += x_move;
-                x = pct_edge(g.X0, vx, g.VW, PCT_X_INC, x_move);
-                y = pct_corr(dy_dx, x, x_start, y_start);
-                x_to_go = g.VW;
-                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-            } else {
-                vy -= y_move;
-                y = pct_edge(g.Y0, vy, g.VH, PCT_Z_INC, y_move);
-                x = pct_corr(dx_dy, y, y_start, x_start);
-                x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-                y_to_go = g.VH;
-            }
-            if (x_to_go == 0) { x_to_go = g.VW; vx += x_move; }
-            if (y_to_go == 0) { y_to_go = g.VH; vy -= y_move; }
         }
-        voxel = vx + (int64_t)vy * C + (int64_t)vz * C * R;
-        outside = (vx >= C) || (vy >= R) || (vz >= S) || (vx < 0) || (vy < 0) || (vz < 0);
-        if (!outside) hit = hull_bit(hull, voxel);
-        end_walk = outside || hit;
-        if (++steps > cap) {
-            hit = 0;
-            end_walk = true;
+        if (axis != 3) w.position(axis, &x, &y, &z);
+    } else {
+        const double delta_yx = fabs(txy);
+        double x_to_go = pct_dist(g.X0, x, PCT_X_INC, w.xm, g.VW, w.vx);
+        double y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, w.ym, g.VH, w.vy);
+        while (!end_walk) {
+            const double y_ext = y_to_go / delta_yx;
+            if (x_to_go <= y_ext) {
+                w.vx += w.xm;
+                x = pct_edge(g.X0, w.vx, g.VW, PCT_X_INC, w.xm);
+                y = pct_corr(w.dy_dx, x, x_start, y_start);
+                x_to_go = g.VW;
+                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, w.ym, g.VH, w.vy);
+            } else {
+                w.vy -= w.ym;
+                y = pct_edge(g.Y0, w.vy, g.VH, PCT_Z_INC, w.ym);
+                x = pct_corr(w.dx_dy, y, y_start, x_start);
+                x_to_go = pct_dist(g.X0, x, PCT_X_INC, w.xm, g.VW, w.vx);
+                y_to_go = g.VH;
+            }
+            if (x_to_go == 0) { x_to_go = g.VW; w.vx += w.xm; }
+            if (y_to_go == 0) { y_to_go = g.VH; w.vy -= w.ym; }
+            end_walk = outside();
+            if (!end_walk) hit = in_hull();
+            end_walk = end_walk || hit;
+            if (++steps > cap) {
+                hit = 0;
+                end_walk = true;
+            }
         }
     }
     if (hit) {
@@ -137,9 +129,9 @@ __device__ int find_endpoint(const DevGeom& g, const uint32_t* __restrict__ hull
         *yo = y;
         *zo = z;
     }
-    *vxo = vx;
-    *vyo = vy;
-    *vzo = vz;
+    *vxo = w.vx;
+    *vyo = w.vy;
+    *vzo = w.vz;
     return hit;
 }
 
@@ -147,7 +139,9 @@ struct H10 {
     float* h[10];
 };
 
-// collect_MLP_endpoints_GPU_nobool, DS.cu:7819-7854.  With `perm`, lane t takes history perm[t]: in
+// collect_MLP_endpoints_GPU_nobool, DS.cu:7819-7854.  Bound by the steps of the walks: 5.8M head histories, 42% of
+// which miss the hull and cross the whole image, 5.9 ms with both walks of every history and the edges formed anew
+// in each step, 4.4 ms with walk.h and the second walk left out where the first found no hull.  With `perm`, lane t takes history perm[t]: in
 // sinogram-bin order the lanes of a wavefront walk nearly the same chords, so their walks to the hull take
 // about as many steps.
 __global__ void k_endpoints(int64_t n, const uint32_t* __restrict__ perm, DevGeom g, const uint32_t* __restrict__ hull,
@@ -160,7 +154,8 @@ __global__ void k_endpoints(int64_t n, const uint32_t* __restrict__ perm, DevGeo
     int vx, vy, vz, vxi, vyi, vzi;
     int entered = find_endpoint(g, hull, hp.h[0][i], hp.h[1][i], hp.h[2][i], hp.h[6][i], hp.h[7][i], &xi, &yi, &zi,
                                 &vx, &vy, &vz, 1);
-    int exited = find_endpoint(g, hull, hp.h[3][i], hp.h[4][i], hp.h[5][i], hp.h[8][i], hp.h[9][i], &xo, &yo, &zo,
+    // a history that does not enter is not kept, wherever it leaves
+    int exited = entered && find_endpoint(g, hull, hp.h[3][i], hp.h[4][i], hp.h[5][i], hp.h[8][i], hp.h[9][i], &xo, &yo, &zo,
                                &vxi, &vyi, &vzi, 0);
     if (entered && exited) {
         first_voxel[i] = (uint32_t)(vx + g.C * vy + g.R * g.C * vz);

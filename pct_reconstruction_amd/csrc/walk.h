@@ -21,6 +21,7 @@ struct Walk3 {
     double xt, yt, zt;
     int kx, ky, kz;
     double ex, ey, ez;
+    double passed;  // the edge passed by the last step
 
     __device__ __forceinline__ void edges(const DevGeom& g)
     {
@@ -56,6 +57,7 @@ struct Walk3 {
     // the distances once an edge at p was passed
     __device__ __forceinline__ void move_x(const DevGeom& g, double p)
     {
+        passed = p;
         const double d = p - xs;
         xt = g.VW;
         yt = fabs(ey - (dy_dx * d + ys));
@@ -63,6 +65,7 @@ struct Walk3 {
     }
     __device__ __forceinline__ void move_y(const DevGeom& g, double p)
     {
+        passed = p;
         const double d = p - ys;
         xt = fabs(ex - (dx_dy * d + xs));
         yt = g.VH;
@@ -70,10 +73,28 @@ struct Walk3 {
     }
     __device__ __forceinline__ void move_z(const DevGeom& g, double p)
     {
+        passed = p;
         const double d = p - zs;
         xt = fabs(ex - (dx_dz * d + xs));
         yt = fabs(ey - (dy_dz * d + ys));
         zt = g.VT;
+    }
+    // the position after a step along `axis`
+    __device__ __forceinline__ void position(int axis, double* x, double* y, double* z) const
+    {
+        if (axis == 0) {
+            *x = passed;
+            *y = dy_dx * (passed - xs) + ys;
+            *z = dz_dx * (passed - xs) + zs;
+        } else if (axis == 1) {
+            *x = dx_dy * (passed - ys) + xs;
+            *y = passed;
+            *z = dz_dy * (passed - ys) + zs;
+        } else {
+            *x = dx_dz * (passed - zs) + xs;
+            *y = dy_dz * (passed - zs) + ys;
+            *z = passed;
+        }
     }
     // One step; the axis moved along.  *full as in resume, *clamped: the z voxel fell below 0 and stays at 0
     // (`at` is then for the caller to set).
