@@ -416,7 +416,7 @@ int pct_tvs_iteration(pct_ctx* ctx, int k);               // NTVS_iteration for 
 int pct_stage_total_variation(pct_ctx* ctx, double* tv);  // TV of ctx->x, fixed-order FP64 sum
 
 // compaction: keep entries with flag != 0 (flag array has ctx->n_hist entries); returns new count
-int pct_compact(pct_ctx* ctx, const uint8_t* keep, int64_t n, int64_t* n_out, bool with_first_voxel);
+int pct_compact(pct_ctx* ctx, const uint8_t* flag, bool drop, int64_t n, int64_t* n_out, bool with_first_voxel);
 // per-history arrays (and their compaction scratch) for n histories
 int pct_ensure_hist_capacity(pct_ctx* ctx, int64_t n);
 int pct_bin_order(pct_ctx* ctx, int64_t n);

@@ -621,7 +621,7 @@ int pct_stage_endpoints(pct_ctx* ctx)
     }
     PCT_CHECK_HIP(ctx, hipGetLastError());
     int64_t kept = 0;
-    PCT_TRY(pct_compact(ctx, ctx->flag, n, &kept, true));  // DS.cu:8286-8294
+    PCT_TRY(pct_compact(ctx, ctx->flag, false, n, &kept, true));  // DS.cu:8286-8294
     ctx->n_hist = kept;
     ctx->n_recon = kept;
     ctx->stage = ST_ENDPOINTS;
