@@ -193,6 +193,9 @@ int pct_ctx_destroy(pct_ctx* ctx)
     pct_free(&ctx->accum64); pct_free(&ctx->accum32); pct_free(&ctx->S); pct_free(&ctx->touched);
     pct_free(&ctx->n_touched); pct_free(&ctx->list_overflow);
     pct_carve_free(ctx);
+    for (auto& b : ctx->scratch) pct_free(&b);
+    pct_free(&ctx->angle_cs);
+    if (ctx->read_h) (void)hipHostFree(ctx->read_h);
     pct_drop_plan_free(&ctx->plan);
     pct_free(&ctx->tvs_G); pct_free(&ctx->tvs_part); pct_free(&ctx->tvs_res);
     if (ctx->tvs_res_h) (void)hipHostFree(ctx->tvs_res_h);
@@ -659,6 +662,19 @@ int pct_drop_iteration_device(int64_t n, const int64_t* offsets, const uint32_t*
 }
 
 }  // extern "C"
+
+int pct_read(pct_ctx* ctx, void* dst, const void* src, size_t bytes)
+{
+    if (bytes <= kReadBytes && !ctx->read_h && hipHostMalloc(&ctx->read_h, kReadBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->read_h = nullptr;
+    }
+    void* to = bytes <= kReadBytes && ctx->read_h ? ctx->read_h : dst;
+    PCT_CHECK_HIP(ctx, hipMemcpyAsync(to, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    PCT_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (to != dst) std::memcpy(dst, to, bytes);
+    return PCT_OK;
+}
 
 int pct_grow_cub(pct_ctx* ctx, size_t need)
 {

@@ -248,6 +248,9 @@ struct pct_ctx {
     uint32_t* u32_c = nullptr;
     uint32_t* u32_d = nullptr;
     void* cub_tmp = nullptr;
+    uint8_t* scratch[6] = {};      // by ScratchSlot
+    void* read_h = nullptr;        // pinned, kReadBytes: where small results land (pct_read)
+    double* angle_cs = nullptr;    // cos and sin of the angle bins, as the binning and as the FBP form them
     size_t cub_tmp_bytes = 0;
     int64_t bin_perm_n = -1;  // u32_d holds the bin order of the first bin_perm_n histories (pct_bin_order)
     int carve_spill = 512;    // LDS count at which a carve visit goes to global memory, 1..512 (PCT_CARVE_SPILL)
@@ -332,14 +335,23 @@ struct pct_ctx {
 };
 
 // allocation helpers
+// A buffer that is there already and holds `count` elements, with at most a quarter and 64 KB to spare, stays: a
+// context that runs its stages again asks for the same sizes, and a free and an allocation took 10 to 60 us each
+// time, 33 times in a reconstruction.
 template <class T>
 int pct_alloc(pct_ctx* ctx, T** p, size_t count)
 {
+    if (count == 0) count = 1;
     if (*p) {
+        hipDeviceptr_t base = nullptr;
+        size_t have = 0;
+        const size_t need = count * sizeof(T);
+        if (hipMemGetAddressRange(&base, &have, (hipDeviceptr_t)*p) == hipSuccess && base == (hipDeviceptr_t)*p &&
+            have >= need && have - need <= need / 4 + (64 << 10))
+            return PCT_OK;
         (void)hipFree(*p);
         *p = nullptr;
     }
-    if (count == 0) count = 1;
     hipError_t e = hipMalloc((void**)p, count * sizeof(T));
     if (e != hipSuccess) {
         ctx->err = std::string("hipMalloc(") + std::to_string(count * sizeof(T)) + " B): " + hipGetErrorString(e);
@@ -354,6 +366,15 @@ void pct_free(T** p)
     if (*p) (void)hipFree(*p);
     *p = nullptr;
 }
+// Scratch of one stage, kept by the context for its next run; every use is on the context's stream, in order.
+enum ScratchSlot { SCR_THRESHOLD, SCR_HULL_BITS, SCR_BLOCK_PROC, SCR_BLOCK_ENTRIES, SCR_BLOCK_SLOTS, SCR_TILE_MARK };
+template <class T>
+int pct_scratch(pct_ctx* ctx, ScratchSlot slot, T** p, size_t count)
+{
+    PCT_TRY(pct_alloc(ctx, &ctx->scratch[slot], count * sizeof(T)));
+    *p = (T*)ctx->scratch[slot];
+    return PCT_OK;
+}
 // A device buffer owned by one stage call: freed when the call returns, on its error paths too.
 template <class T>
 struct pct_tmp {
@@ -366,6 +387,11 @@ struct pct_tmp {
 
 DevGeom pct_geom(const pct_params& P);
 void pct_carve_free(pct_ctx* ctx);              // the carve's scratch
+// The first `bytes` at src on the device, once the stream is done: through pinned memory where they are few (a copy to
+// pageable memory stages and waits for itself, 10 us more).
+constexpr size_t kReadBytes = 4096;
+int pct_read(pct_ctx* ctx, void* dst, const void* src, size_t bytes);
+int pct_angle_table(pct_ctx* ctx);            // ctx->angle_cs, once
 int pct_grow_cub(pct_ctx* ctx, size_t need);  // library scratch of at least `need` bytes
 
 // host-side tables (tables.cpp)

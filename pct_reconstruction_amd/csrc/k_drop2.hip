@@ -814,8 +814,7 @@ int build_slices(pct_ctx* ctx, DropPlan& D)
     tb = ctx->cub_tmp_bytes;
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, tb, w, D.sell_off, (int)(NS + 1), s));
     uint64_t total = 0;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&total, D.sell_off + NS, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &total, D.sell_off + NS, sizeof(uint64_t)));
     PCT_TRY(grow(ctx, &D.sell, &D.cap_sell, (int64_t)total + 1));
     if (NS > 0)
         hipLaunchKernelGGL(k_slice_fill, dim3(grid), dim3(kWave), 0, s, NS, chunk, nb, D.slice_blocks, D.t_off,
@@ -927,8 +926,7 @@ int transpose_group_buckets(pct_ctx* ctx, DropPlan& D, const DropPlan::Group& g,
     PCT_CHECK_HIP(ctx, hipGetLastError());
     uint32_t nr = 0, total = 0;
     PCT_CHECK_HIP(ctx, hipMemcpyAsync(&nr, D.bk_roff + nbk, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&total, D.bk_off + nbk, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &total, D.bk_off + nbk, sizeof(uint32_t)));
     if ((int64_t)total != E || nr < 1 || (int64_t)nr > E) {
         ctx->err = "DROP bucket transposition: entry or run count out of range in a group";
         return PCT_E_LIMIT;
@@ -994,23 +992,20 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
         const int64_t proc = P.quirk_a3_drop_floor ? (m / P.histories_per_block) * P.histories_per_block : m;
         proc_raw[rb] = proc > 0 ? (int32_t)proc : 0;
     }
-    pct_tmp<int32_t> proc_buf;
-    pct_tmp<int64_t> e_buf;
-    PCT_TRY(pct_alloc(ctx, &proc_buf.p, n_raw + 1));
-    PCT_TRY(pct_alloc(ctx, &e_buf.p, n_raw + 1));
-    const int32_t* proc_dev = proc_buf.p;
-    int64_t* e_dev = e_buf.p;
+    int32_t* proc_dev = nullptr;
+    int64_t* e_dev = nullptr;
+    PCT_TRY(pct_scratch(ctx, SCR_BLOCK_PROC, &proc_dev, n_raw + 1));
+    PCT_TRY(pct_scratch(ctx, SCR_BLOCK_ENTRIES, &e_dev, n_raw + 1));
     std::vector<int64_t> e_raw(n_raw > 0 ? n_raw : 1, 0);
     if (n_raw > 0) {
-        PCT_CHECK_HIP(ctx, hipMemcpyAsync(proc_buf.p, proc_raw.data(), n_raw * sizeof(int32_t), hipMemcpyHostToDevice, s));
+        PCT_CHECK_HIP(ctx, hipMemcpyAsync(proc_dev, proc_raw.data(), n_raw * sizeof(int32_t), hipMemcpyHostToDevice, s));
         if (pipe)  // list capacities bound the entries until the lists exist: groups and allocations use them
             hipLaunchKernelGGL(k_block_caps, dim3(grid_for(n_raw)), dim3(kBlock), 0, s, n_raw, BS, proc_dev,
                                ctx->list_off, e_dev);
         else
             hipLaunchKernelGGL(k_block_entries, dim3((unsigned)n_raw), dim3(256), 0, s, BS, proc_dev, ctx->list_cnt,
                                P.min_mlp_length, e_dev);
-        PCT_CHECK_HIP(ctx, hipMemcpyAsync(e_raw.data(), e_dev, n_raw * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+        PCT_TRY(pct_read(ctx, e_raw.data(), e_dev, n_raw * sizeof(int64_t)));
     }
     int64_t total = 0, max_proc = 0;
     for (int64_t rb = 0; rb < n_raw; rb++) {
@@ -1271,8 +1266,7 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
             PCT_CHECK_HIP(ctx, hipcub::DeviceRunLengthEncode::Encode(ctx->cub_tmp, tb, D.keys_sorted, D.keys, D.runs,
                                                                      D.n_runs, (int)E, s));
             // the run count sizes the scan and the runs kernel
-            PCT_CHECK_HIP(ctx, hipMemcpyAsync(&n_runs_h[gi], D.n_runs, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-            PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+            PCT_TRY(pct_read(ctx, &n_runs_h[gi], D.n_runs, sizeof(uint32_t)));
             const int64_t nr = (int64_t)n_runs_h[gi];
             if (nr < 1 || nr > E) {
                 ctx->err = "DROP transposition: run count out of range in a group";
@@ -1319,8 +1313,6 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
         if (bricks) D.vox_b_ready = true;
     }
     PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
-    pct_free(&proc_buf.p);
-    pct_free(&e_buf.p);
     // per block: its runs [run_start, next run_start) within the group
     for (auto& bk : D.blocks) {
         const DropPlan::Group& g = D.groups[bk.group];
@@ -1557,8 +1549,7 @@ int pct_stage_residual(pct_ctx* ctx, double* norm)
         PCT_CHECK_HIP(ctx, hipcub::DeviceReduce::Sum(ctx->cub_tmp, need, ctx->res_r2, out, n, s));
     }
     double h = 0.0;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&h, out, sizeof(double), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &h, out, sizeof(double)));
     *norm = std::sqrt(h);
     return PCT_OK;
 }

@@ -974,8 +974,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
     tb = ctx->cub_tmp_bytes;
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, tb, W.nseg, W.q0, (int)(H + 1), s));
     uint32_t Q = 0;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&Q, W.q0 + H, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &Q, W.q0 + H, sizeof(uint32_t)));
     if (Q > (1u << 30)) return PCT_OK;
     G.segs = Q;
     G.n_runs = 0;
@@ -1008,8 +1007,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
     PCT_CHECK_HIP(ctx, hipcub::DeviceRunLengthEncode::Encode(ctx->cub_tmp, tb, keys_sorted, W.keys, W.runs, W.n_runs,
                                                              (int)Q, s));
     uint32_t nr = 0, lim[kLimits] = {};
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&nr, W.n_runs, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &nr, W.n_runs, sizeof(uint32_t)));
     if (nr < 1 || nr > Q) {
         ctx->err = "DROP tiles: run count out of range in a group";
         return PCT_E_LIMIT;
@@ -1039,8 +1037,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
     PCT_CHECK_HIP(ctx, hipcub::DeviceReduce::Max(ctx->cub_tmp, tb, W.runs, W.limits + 1, (int)nr, s));
     tb = ctx->cub_tmp_bytes;
     PCT_CHECK_HIP(ctx, hipcub::DeviceReduce::Max(ctx->cub_tmp, tb, entries, W.limits + 2, (int)nr, s));
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(lim, W.limits, sizeof(lim), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, lim, W.limits, sizeof(lim)));
     if (lim[1] > kMaxSeg || lim[2] > kMaxEnt || lim[2 + kClasses] < nr) return PCT_OK;
     const uint32_t* classes = lim + 3;
     PCT_CHECK_HIP(ctx, hipFuncSetAttribute((const void*)k_tile_fill, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1062,8 +1059,7 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
         PCT_CHECK_HIP(ctx, hipGetLastError());
         uint64_t total = 0;
         PCT_CHECK_HIP(ctx, hipMemcpyAsync(&total, W.cursor, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-        PCT_CHECK_HIP(ctx, hipMemcpyAsync(lim, W.limits, sizeof(lim), hipMemcpyDeviceToHost, s));
-        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+        PCT_TRY(pct_read(ctx, lim, W.limits, sizeof(lim)));
         if (lim[0] || total >= (1ull << 32)) return PCT_OK;
         if ((int64_t)total * 64 + kSlack <= G.cap_words) {
             *fits = true;
@@ -1163,38 +1159,35 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
         const int64_t p = P.quirk_a3_drop_floor ? (m / P.histories_per_block) * P.histories_per_block : m;
         proc[rb] = p > 0 ? (int32_t)p : 0;
     }
-    pct_tmp<int32_t> proc_buf;
-    pct_tmp<int64_t> cap_buf;
-    PCT_TRY(pct_alloc(ctx, &proc_buf.p, n_raw));
-    PCT_TRY(pct_alloc(ctx, &cap_buf.p, n_raw));
+    int32_t* proc_dev = nullptr;
+    int64_t *cap_dev = nullptr, *slot_dev = nullptr;
+    PCT_TRY(pct_scratch(ctx, SCR_BLOCK_PROC, &proc_dev, n_raw + 1));
+    PCT_TRY(pct_scratch(ctx, SCR_BLOCK_ENTRIES, &cap_dev, n_raw + 1));
+    PCT_TRY(pct_scratch(ctx, SCR_BLOCK_SLOTS, &slot_dev, n_raw + 1));
     std::vector<int64_t> cap(n_raw), first_slot(n_raw);
-    pct_tmp<int64_t> slot_buf;
-    PCT_TRY(pct_alloc(ctx, &slot_buf.p, n_raw));
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(proc_buf.p, proc.data(), n_raw * sizeof(int32_t), hipMemcpyHostToDevice, s));
+    PCT_CHECK_HIP(ctx, hipMemcpyAsync(proc_dev, proc.data(), n_raw * sizeof(int32_t), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_tile_block_caps, dim3(grid_for(n_raw)), dim3(kBlock), 0, s, n_raw, BS, n,
-                       ctx->list_off, cap_buf.p, slot_buf.p);
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(cap.data(), cap_buf.p, n_raw * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(first_slot.data(), slot_buf.p, n_raw * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+                       ctx->list_off, cap_dev, slot_dev);
+    PCT_CHECK_HIP(ctx, hipMemcpyAsync(cap.data(), cap_dev, n_raw * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    PCT_TRY(pct_read(ctx, first_slot.data(), slot_dev, n_raw * sizeof(int64_t)));
     int64_t slots = 0;
     for (int64_t rb = 0; rb < n_raw; rb++) slots += cap[rb];
     const int64_t nb_est = std::max<int64_t>(1, n / BS);
     // The rule: list slots of a block per tile that the paths reach (see kMinSlots)
     double density = 0.0;
     if (ctx->drop_tiles != 1) {
-        pct_tmp<uint8_t> mark;
-        PCT_TRY(pct_alloc(ctx, &mark.p, g.nt));
-        PCT_CHECK_HIP(ctx, hipMemsetAsync(mark.p, 0, g.nt, s));
+        uint8_t* mark = nullptr;
+        PCT_TRY(pct_scratch(ctx, SCR_TILE_MARK, &mark, g.nt));
+        PCT_CHECK_HIP(ctx, hipMemsetAsync(mark, 0, g.nt, s));
         SampleArgs a{n, (n + kSample - 1) / kSample, g, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, pct_geom(P),
                      ctx->list_off, ctx->list_cnt, ctx->list_vox};
         if (pipe) {
             a.x0 = ctx->h[0], a.y0 = ctx->h[1], a.z0 = ctx->h[2];
             a.x1 = ctx->h[3], a.y1 = ctx->h[4], a.z1 = ctx->h[5];
         }
-        hipLaunchKernelGGL(k_tile_sample, dim3(grid_for((n + a.every - 1) / a.every)), dim3(kBlock), 0, s, a, mark.p);
+        hipLaunchKernelGGL(k_tile_sample, dim3(grid_for((n + a.every - 1) / a.every)), dim3(kBlock), 0, s, a, mark);
         std::vector<uint8_t> m(g.nt);
-        PCT_CHECK_HIP(ctx, hipMemcpyAsync(m.data(), mark.p, g.nt, hipMemcpyDeviceToHost, s));
-        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+        PCT_TRY(pct_read(ctx, m.data(), mark, g.nt));
         int64_t reached = 0;
         for (uint8_t v : m) reached += v;
         density = (double)slots / nb_est / (double)std::max<int64_t>(1, reached);
@@ -1289,7 +1282,7 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
         if (pipe) PCT_CHECK_HIP(ctx, hipStreamWaitEvent(s, q.ev[gi + 1], 0));
         const int64_t rb0 = gr.hist_begin / BS;
         CutArgs a{gr.hist_begin, gr.hist_end - gr.hist_begin, BS, rb0, slot0[gi], g, tile_bits, P.min_mlp_length,
-                  proc_buf.p, nullptr, ctx->list_off, ctx->list_cnt, ctx->list_vox, ctx->chord, ctx->wepl};
+                  proc_dev, nullptr, ctx->list_off, ctx->list_cnt, ctx->list_vox, ctx->chord, ctx->wepl};
         T.groups[gi].entries_hint = gr.entries;
         PCT_TRY(build_group(ctx, T, T.groups[gi], a, bin_bits, T.totals + rb0, &fits));
     }
@@ -1318,8 +1311,7 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
     PCT_CHECK_HIP(ctx, hipMemcpyAsync(T.block_of, block_of.data(), n_raw * sizeof(int32_t), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_tile_block_seg, dim3(grid_for(n_raw)), dim3(kBlock), 0, s, n_raw, BS, T.block_of, T.rows, T.totals);
     PCT_CHECK_HIP(ctx, hipMemcpyAsync(used.data(), T.used, g.nt, hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(totals.data(), T.totals, n_raw * sizeof(BlockTotals), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, totals.data(), T.totals, n_raw * sizeof(BlockTotals)));
     std::vector<uint32_t> index_of(g.nt, 0);
     int64_t U = 0;
     for (uint32_t k = 0; k < g.nt; k++)

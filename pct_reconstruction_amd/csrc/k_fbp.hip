@@ -174,18 +174,9 @@ int pct_stage_fbp(pct_ctx* ctx)
                        ctx->sino_filtered, T, P.angular_bins, P.v_bins, P.t_bin_size, P.v_bin_size, P.source_radius,
                        P.pi, P.fbp_filter_type, P.ram_lak_tau);
     PCT_CHECK_HIP(ctx, hipGetLastError());
-    // cos/sin of bin_angle = angle_bin * delta (DS.cu:6362-6364)
     const double delta = P.angular_bin_size * (P.pi / 180.0);
-    std::vector<double> cs(2 * P.angular_bins);
-    for (int a = 0; a < P.angular_bins; a++) {
-        double ba = a * delta;
-        cs[a] = std::cos(ba);
-        cs[P.angular_bins + a] = std::sin(ba);
-    }
-    pct_tmp<double> cs_buf;
-    PCT_TRY(pct_alloc(ctx, &cs_buf.p, cs.size()));
-    const double* d_cs = cs_buf.p;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(cs_buf.p, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice, s));
+    PCT_TRY(pct_angle_table(ctx));
+    const double* d_cs = ctx->angle_cs + 2 * P.angular_bins;
     BPArgs a;
     a.T = T;
     a.V = P.v_bins;
@@ -207,8 +198,6 @@ int pct_stage_fbp(pct_ctx* ctx)
     hipLaunchKernelGGL(k_backproject, dim3(grid_for(P.num_voxels)), dim3(kBlock), 0, s, a, ctx->sino_filtered, d_cs,
                        ctx->fbp);
     PCT_CHECK_HIP(ctx, hipGetLastError());
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
-    pct_free(&cs_buf.p);
     PCT_TRY(pct_median_filter_fbp(ctx));  // FBP(), DS.cu:6150-6166 (x0 only)
     if (P.hull_type == PCT_HULL_FBP) PCT_TRY(pct_fbp_hull(ctx));
     ctx->stage = ST_FBP;

@@ -670,8 +670,7 @@ int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gat
         scan = ctx->cub_tmp_bytes;
         PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, scan, W.cap, W.off, (int)(m + 1), s));
         uint32_t total = 0;
-        PCT_CHECK_HIP(ctx, hipMemcpyAsync(&total, W.off + m, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+        PCT_TRY(pct_read(ctx, &total, W.off + m, sizeof(uint32_t)));
         if (total > 0) {
             uint32_t *keys, *sorted_keys, *start = W.tiles, *first_chunk = W.tiles + tiles + 1;
             uint64_t *vals, *sorted_vals;
@@ -781,14 +780,11 @@ int pct_stage_hull_finish(pct_ctx* ctx)
     }
     if (P.sm_on) {
         PCT_TRY(pct_alloc(ctx, &ctx->sm_hull, NV));
-        pct_tmp<int32_t> thr_buf;
-        PCT_TRY(pct_alloc(ctx, &thr_buf.p, P.slices));
-        int32_t* thr = thr_buf.p;
+        int32_t* thr = nullptr;
+        PCT_TRY(pct_scratch(ctx, SCR_THRESHOLD, &thr, P.slices));
         hipLaunchKernelGGL(k_sm_threshold, dim3(P.slices), dim3(kBlock), 0, s, g, ctx->sm_counts, thr);
         hipLaunchKernelGGL(k_sm_edge, dim3(grid_for(NV)), dim3(kBlock), 0, s, g, ctx->sm_counts, thr, ctx->sm_hull,
                            P.sm_scale_threshold);
-        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
-        pct_free(&thr_buf.p);
     }
     PCT_CHECK_HIP(ctx, hipGetLastError());
     ctx->stage = ST_HULLS;

@@ -610,13 +610,13 @@ int pct_stage_endpoints(pct_ctx* ctx)
         PCT_TRY(pct_bin_order(ctx, n));
         perm = ctx->u32_d;
     }
-    pct_tmp<uint32_t> bits;
+    uint32_t* bits = nullptr;
     if (n > 0) {
         const int64_t NV = P.num_voxels, words = (NV + 31) / 32;
-        PCT_TRY(pct_alloc(ctx, &bits.p, words));
+        PCT_TRY(pct_scratch(ctx, SCR_HULL_BITS, &bits, words));
         hipLaunchKernelGGL(k_hull_bits, dim3(grid_for(words)), dim3(kBlock), 0, s, NV,
-                           ctx->hull_endpoints ? ctx->hull_endpoints : ctx->hull, bits.p);
-        hipLaunchKernelGGL(k_endpoints, dim3(grid_for(n)), dim3(kBlock), 0, s, n, perm, g, bits.p, hp,
+                           ctx->hull_endpoints ? ctx->hull_endpoints : ctx->hull, bits);
+        hipLaunchKernelGGL(k_endpoints, dim3(grid_for(n)), dim3(kBlock), 0, s, n, perm, g, bits, hp,
                            ctx->first_voxel, ctx->flag);
     }
     PCT_CHECK_HIP(ctx, hipGetLastError());
@@ -719,8 +719,7 @@ int pct_stage_build_lists(pct_ctx* ctx)
     }
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, need, capv, ctx->list_off, n + 1, s));
     int64_t total = 0;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&total, ctx->list_off + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &total, ctx->list_off + n, sizeof(int64_t)));
     if (total > ctx->list_cap) {
         PCT_TRY(pct_alloc(ctx, &ctx->list_vox, total));
         ctx->list_cap = total;
@@ -786,8 +785,7 @@ int pct_stage_build_lists(pct_ctx* ctx)
         (void)hipEventDestroy(e1);
     }
     int32_t overflow = 0;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&overflow, ctx->list_overflow, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &overflow, ctx->list_overflow, sizeof(int32_t)));
     if (overflow) {
         ctx->err = "MLP list capacity exceeded (code " + std::to_string(overflow) + ")";
         ctx->plan.ready = false;  // a plan built with the lists holds them
@@ -801,8 +799,7 @@ int pct_stage_build_lists(pct_ctx* ctx)
         hipLaunchKernelGGL(k_count_entries, dim3(pct_grid_capped(n, kBlock, 2048)), dim3(kBlock), 0, s, n,
                            ctx->list_cnt, d_total);
     unsigned long long listed = 0;
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(&listed, d_total, sizeof(listed), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, &listed, d_total, sizeof(listed)));
     ctx->list_entries = (int64_t)listed;
     ctx->stage = ST_LISTS;
     if (pipe) return PCT_OK;  // the plan was built with the lists

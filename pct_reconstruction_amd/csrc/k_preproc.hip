@@ -249,6 +249,11 @@ __device__ __forceinline__ double wrap_pi(double a, double PI)
     return a;
 }
 
+// doubles as two arrays of words
+struct Words {
+    uint32_t *lo, *hi;
+};
+
 // The per-history inputs of the bin statistics in bin order (j = position in the sorted order): in-range
 // flag, WEPL and the two wrapped angle differences, so that the three passes of k_bin_stats stream
 // contiguous memory instead of gathering through the order.
@@ -256,7 +261,7 @@ __global__ void k_bin_gather(int64_t n, const uint32_t* __restrict__ perm, const
                              const float* __restrict__ wepl, const float* __restrict__ xya_e,
                              const float* __restrict__ xza_e, const float* __restrict__ xya_x,
                              const float* __restrict__ xza_x, double PI, uint8_t* __restrict__ g_ir,
-                             float* __restrict__ g_w, double* __restrict__ g_ut, double* __restrict__ g_uv)
+                             float* __restrict__ g_w, double* __restrict__ g_ut, Words g_uv)
 {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
@@ -264,7 +269,9 @@ __global__ void k_bin_gather(int64_t n, const uint32_t* __restrict__ perm, const
     g_ir[j] = in_range[i];
     g_w[j] = wepl[i];
     g_ut[j] = wrap_pi((double)(xya_x[i] - xya_e[i]), PI);
-    g_uv[j] = wrap_pi((double)(xza_x[i] - xza_e[i]), PI);
+    const double uv = wrap_pi((double)(xza_x[i] - xza_e[i]), PI);
+    g_uv.lo[j] = (uint32_t)__double2loint(uv);
+    g_uv.hi[j] = (uint32_t)__double2hiint(uv);
 }
 
 // One lane per bin: binning sums (DS.cu:5518-5546), calculate_means_GPU (:5644), the squared
@@ -277,7 +284,7 @@ constexpr int kStatChunk = 1024;
 __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restrict__ off,
                                                   const uint32_t* __restrict__ perm, const uint8_t* __restrict__ g_ir,
                                                   const float* __restrict__ g_w, const double* __restrict__ g_ut,
-                                                  const double* __restrict__ g_uv, int32_t* counts_pre, float* m_w,
+                                                  Words g_uv, int32_t* counts_pre, float* m_w,
                                                   float* m_ut, float* m_uv, float* s_w, float* s_ut, float* s_uv,
                                                   int32_t* counts_post, float* sinogram, uint8_t* failed, float k,
                                                   int quirk_a1)
@@ -297,7 +304,7 @@ __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restr
 #pragma unroll 4
                 for (int j = threadIdx.x; j < m; j += 64) {
                     l_ut[j] = g_ut[c0 + j];
-                    l_uv[j] = g_uv[c0 + j];
+                    l_uv[j] = __hiloint2double((int)g_uv.hi[c0 + j], (int)g_uv.lo[c0 + j]);
                     l_w[j] = g_w[c0 + j];
                     l_ir[j] = g_ir[c0 + j];
                 }
@@ -406,8 +413,7 @@ int pct_compact(pct_ctx* ctx, const uint8_t* flag, bool drop, int64_t n, int64_t
         hipLaunchKernelGGL(k_compact<13>, dim3(grid_for(n)), dim3(kBlock), 0, s, n, flag, kept, ctx->pos, c);
     }
     PCT_CHECK_HIP(ctx, hipGetLastError());
-    PCT_CHECK_HIP(ctx, hipMemcpyAsync(n_out, ctx->pos + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    PCT_TRY(pct_read(ctx, n_out, ctx->pos + n, sizeof(int64_t)));
     return PCT_OK;
 }
 
@@ -510,6 +516,32 @@ int pct_ensure_hist_capacity(pct_ctx* ctx, int64_t n)
 
 int pct_carve_counts(pct_ctx* ctx);  // k_hull.hip
 
+int pct_angle_table(pct_ctx* ctx)
+{
+    if (ctx->angle_cs) return PCT_OK;
+    const pct_params& P = ctx->P;
+    const int A = P.angular_bins;
+    const double delta = P.angular_bin_size * (P.pi / 180.0);
+    std::vector<double> cs(4 * (size_t)A);
+    for (int a = 0; a < A; a++) {
+        // angle_bin * ANGULAR_BIN_SIZE * ANGLE_TO_RADIANS (DS.cu:5506), and bin_angle = angle_bin * delta (:6362-6364)
+        const double binning = a * P.angular_bin_size * (P.pi / 180.0), fbp = a * delta;
+        cs[a] = std::cos(binning);
+        cs[A + a] = std::sin(binning);
+        cs[2 * A + a] = std::cos(fbp);
+        cs[3 * A + a] = std::sin(fbp);
+    }
+    double* d = nullptr;
+    PCT_TRY(pct_alloc(ctx, &d, cs.size()));
+    if (hipMemcpy(d, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+        pct_free(&d);
+        ctx->err = "angle table: copy failed";
+        return PCT_E_HIP;
+    }
+    ctx->angle_cs = d;
+    return PCT_OK;
+}
+
 int pct_stage_intersect_bin_carve(pct_ctx* ctx)
 {
     const pct_params& P = ctx->P;
@@ -526,23 +558,12 @@ int pct_stage_intersect_bin_carve(pct_ctx* ctx)
     if (n > 0) {
         hipLaunchKernelGGL(k_intersections, dim3(g), dim3(kBlock), 0, s, n, r, o, ctx->wepl, ctx->gantry, missed,
                            P.recon_cyl_radius, P.recon_cyl_height, P.pi / 180.0);
-        // angle-bin centres: angle_bin * ANGULAR_BIN_SIZE * ANGLE_TO_RADIANS (DS.cu:5506)
-        std::vector<double> cs(2 * P.angular_bins);
-        for (int a = 0; a < P.angular_bins; a++) {
-            double angle = a * P.angular_bin_size * (P.pi / 180.0);
-            cs[a] = std::cos(angle);
-            cs[P.angular_bins + a] = std::sin(angle);
-        }
-        pct_tmp<double> cs_buf;
-        PCT_TRY(pct_alloc(ctx, &cs_buf.p, cs.size()));
-        const double* d_cs = cs_buf.p;
-        PCT_CHECK_HIP(ctx, hipMemcpyAsync(cs_buf.p, cs.data(), cs.size() * sizeof(double), hipMemcpyHostToDevice, s));
+        PCT_TRY(pct_angle_table(ctx));
+        const double* d_cs = ctx->angle_cs;
         hipLaunchKernelGGL(k_binning, dim3(g), dim3(kBlock), 0, s, n, o, missed, ctx->bin_num, ctx->in_range, d_cs,
                            d_cs + P.angular_bins, P.pi, P.angular_bin_size, P.t_bin_size, P.v_bin_size, P.t_bins,
                            P.v_bins, P.angular_bins);
         PCT_CHECK_HIP(ctx, hipGetLastError());
-        PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
-        pct_free(&cs_buf.p);
     }
     // keep histories that traversed the reconstruction volume (DS.cu:5429-5449)
     int64_t kept = 0;
@@ -580,18 +601,16 @@ int pct_stage_stats_and_cuts(pct_ctx* ctx)
     hipLaunchKernelGGL(k_bin_offsets, dim3(grid_for(NB + 1)), dim3(kBlock), 0, s, n, NB, ctx->u32_b, ctx->bin_off);
     uint8_t* failed = ctx->flag;
     if (n > 0) PCT_CHECK_HIP(ctx, hipMemsetAsync(failed, 0, n, s));
-    pct_tmp<uint8_t> g_ir;
-    pct_tmp<float> g_w;
-    pct_tmp<double> g_ut, g_uv;
-    PCT_TRY(pct_alloc(ctx, &g_ir.p, n > 0 ? n : 1));
-    PCT_TRY(pct_alloc(ctx, &g_w.p, n > 0 ? n : 1));
-    PCT_TRY(pct_alloc(ctx, &g_ut.p, n > 0 ? n : 1));
-    PCT_TRY(pct_alloc(ctx, &g_uv.p, n > 0 ? n : 1));
+    // the gathered inputs lie in columns that the compaction at the end overwrites and in scratch of the bin order
+    uint8_t* g_ir = ctx->u8_tmp;
+    float* g_w = ctx->wepl_tmp;
+    double* g_ut = (double*)ctx->pos;
+    const Words g_uv{ctx->u32_a, ctx->u32_c};
     if (n > 0)
         hipLaunchKernelGGL(k_bin_gather, dim3(g), dim3(kBlock), 0, s, n, perm, ctx->in_range, ctx->wepl, ctx->h[6],
-                           ctx->h[7], ctx->h[8], ctx->h[9], P.pi, g_ir.p, g_w.p, g_ut.p, g_uv.p);
-    hipLaunchKernelGGL(k_bin_stats, dim3(pct_grid_for(NB, 64)), dim3(64), 0, s, NB, ctx->bin_off, perm, g_ir.p, g_w.p,
-                       g_ut.p, g_uv.p, ctx->counts_pre, ctx->mean[0], ctx->mean[1], ctx->mean[2], ctx->stddev[0],
+                           ctx->h[7], ctx->h[8], ctx->h[9], P.pi, g_ir, g_w, g_ut, g_uv);
+    hipLaunchKernelGGL(k_bin_stats, dim3(pct_grid_for(NB, 64)), dim3(64), 0, s, NB, ctx->bin_off, perm, g_ir, g_w,
+                       g_ut, g_uv, ctx->counts_pre, ctx->mean[0], ctx->mean[1], ctx->mean[2], ctx->stddev[0],
                        ctx->stddev[1], ctx->stddev[2], ctx->counts_post, ctx->sinogram, failed,
                        (float)P.sigmas_2_keep, P.quirk_a1_bin0);
     PCT_CHECK_HIP(ctx, hipGetLastError());
