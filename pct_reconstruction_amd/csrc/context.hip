@@ -148,6 +148,10 @@ int pct_ctx_create(const pct_params* p, int device, pct_ctx** out)
         int b = std::atoi(e);
         if (b >= -1 && b <= 64) ctx->mlp_blocks_per_cu = b;
     }
+    if (const char* e = std::getenv("PCT_MLP_LANES")) {
+        int l = std::atoi(e);
+        if (l == 1 || l == 4 || l == 16) ctx->mlp_lanes = l;
+    }
     if (const char* e = std::getenv("PCT_DROP_GROUP_ENTRIES")) {
         long long g = std::atoll(e);
         if (g >= 1 && g <= (1ll << 30)) ctx->drop_group_entries = g;

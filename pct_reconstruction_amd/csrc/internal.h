@@ -255,6 +255,7 @@ struct pct_ctx {
     int64_t bin_perm_n = -1;  // u32_d holds the bin order of the first bin_perm_n histories (pct_bin_order)
     int carve_spill = 512;    // LDS count at which a carve visit goes to global memory, 1..512 (PCT_CARVE_SPILL)
     int carve_table = 8192;   // LDS hash slots of the fused carve (4096, 8192, 16384); 0: one walk per method (PCT_CARVE_TABLE)
+    int mlp_lanes = 0;         // lanes per history of the MLP list kernels: 0 by rule, 1, 4, 16 (PCT_MLP_LANES)
     int carve_tiles = -1;      // hull carving by tiles: -1 by rule, 0 never, 1 always (PCT_CARVE_TILES)
     CarveScratch carve;
     int carve_line_order = 1;  // hull carving in chord-line order (both directions of a line together; PCT_CARVE_LINES)

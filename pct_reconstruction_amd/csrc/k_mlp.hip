@@ -4,7 +4,7 @@
 // voxel (find_MLP_endpoints_GPU, DS.cu:7581-7773), the histories in sinogram-bin order and the hull
 // as a bit mask.
 //
-// MLP lists: a one-history-per-lane kernel.  The Sigma_1 terms of every u-step (they depend only on
+// MLP lists: a history per lane, or, where there are few, per 4 or 16 lanes that take steps in turn.  The Sigma_1 terms of every u-step (they depend only on
 // the step number) are precomputed on the host in FP64 and staged in LDS at kernel start; per step a
 // lane reads them from LDS, one scattering coefficient for its Sigma_2 from the FP64 table in HBM/L2,
 // and does the 2x2 inversions and the t/v solve in FP64 exactly as find_MLP_path_GPU_tabulated
@@ -282,6 +282,37 @@ struct ListWriter {
     }
 };
 
+// A list written by the G lanes of a group, which take G consecutive steps at a time: a voxel is listed if it is in
+// the image and differs from the one before it in the image, which is the last listed one.
+template <int G>
+struct GroupList {
+    uint32_t* vox;  // the history's list
+    int64_t cap, cnt;
+    uint32_t last;
+    int l;
+    __device__ __forceinline__ uint32_t group(uint64_t ballot) const
+    {
+        return (uint32_t)(ballot >> ((threadIdx.x & 63u) & ~(unsigned)(G - 1))) & ((1u << G) - 1u);
+    }
+    // the group's next steps, the active ones first; false when the list is full
+    __device__ __forceinline__ bool put(bool in_image, uint32_t v)
+    {
+        const uint32_t in = group(__ballot(in_image)), before = in & ((1u << l) - 1u);
+        const uint32_t left = __shfl(v, before ? 31 - __clz((int)before) : l, G);
+        const bool listed = in_image && v != (before ? left : last);
+        const uint32_t put = group(__ballot(listed));
+        const int64_t at = cnt + __popc(put & ((1u << l) - 1u));
+        if (listed && at < cap) vox[at] = v;
+        const uint32_t end = __shfl(v, in ? 31 - __clz((int)in) : l, G);
+        last = in ? end : last;
+        cnt += __popc(put);
+        const bool room = cnt <= cap;
+        cnt = room ? cnt : cap;
+        return room;
+    }
+};
+
+template <int G>
 __global__ void __launch_bounds__(kBlock) k_mlp_lists(int64_t n, MlpArgs a, H10 hp, const uint32_t* __restrict__ first,
                                                       const double* __restrict__ sin_t,
                                                       const double* __restrict__ cos_t,
@@ -293,15 +324,16 @@ __global__ void __launch_bounds__(kBlock) k_mlp_lists(int64_t n, MlpArgs a, H10 
                                                       int32_t* overflow)
 {
     extern __shared__ double lds_terms[];  // n_steps x 6
-    __shared__ uint32_t list_buf[16 * kBlock];
+    __shared__ uint32_t list_buf[G == 1 ? 16 * kBlock : 1];
     for (int k = threadIdx.x; k < a.n_steps; k += blockDim.x) {
 #pragma unroll
         for (int c = 0; c < 6; c++) lds_terms[k * 6 + c] = step_terms[k * 8 + c];
     }
     __syncthreads();
     const DevGeom& g = a.g;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const int l = threadIdx.x & (G - 1);
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x / G;
+    for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; i < n; i += stride) {
         const double x_in = hp.h[0][i], y_in = hp.h[1][i], z_in = hp.h[2][i];
         const double x_out = hp.h[3][i], y_out = hp.h[4][i], z_out = hp.h[5][i];
         const double xz_entry = hp.h[7][i], xz_exit = hp.h[9][i];
@@ -318,15 +350,11 @@ __global__ void __launch_bounds__(kBlock) k_mlp_lists(int64_t n, MlpArgs a, H10 
         const int64_t base = off[i], capn = off[i + 1] - off[i];
         uint32_t last = first[i];
         int64_t cnt = 1;
-        ListWriter w(vox, list_buf, base);
-        w.put(last);
-        chord[i] = chord_length(g.PI, g.VW, g.VT, STEP, (f.xy_entry + f.xy_exit) / 2.0, (xz_entry + xz_exit) / 2.0);
+        const double L = chord_length(g.PI, g.VW, g.VT, STEP, (f.xy_entry + f.xy_exit) / 2.0, (xz_entry + xz_exit) / 2.0);
+        if (l == 0) chord[i] = L;
         int k = 0;
-        while (depth > STEP) {
-            if (k >= a.n_steps || (int64_t)s2 >= a.n_coeff) {
-                atomicOr(overflow, 1);
-                break;
-            }
+        // the voxel of step k at `depth` before the exit and u_shifted along the path
+        auto voxel_of = [&](int k, unsigned s2, double depth, double u_shifted) -> int64_t {
             const double* row = lds_terms + k * 6;
             const double u1_12 = row[0], u1_23 = row[1], u1_34 = row[2];
             const double S1I0 = row[3], S1I1 = row[4], S1I2 = row[5];
@@ -349,28 +377,64 @@ __global__ void __launch_bounds__(kBlock) k_mlp_lists(int64_t n, MlpArgs a, H10 
             sc0 = S1I0 * z_in + c3;
             sc1 = depth * c3 + S2I2 * V2_1 - S2I1 * z_out - S1I1 * z_in;
             double v_1 = (ft3 * sc0 - ft1 * sc1) / detft;
-            u_shifted += STEP;
             double x_1 = f.cos_t * u_shifted - f.sin_t * t_1;
             double y_1 = f.sin_t * u_shifted + f.cos_t * t_1;
             int vx = pct_calc_voxel(g.X0, x_1, g.VW);
             int vy = pct_calc_voxel(g.Y0, y_1, g.VH);
             int vz = pct_calc_voxel(g.Z0, v_1, g.VT);
-            int64_t voxel = vx + (int64_t)vy * g.C + (int64_t)vz * g.C * g.R;
-            if (voxel != (int64_t)last && voxel < g.NV) {
-                if (cnt >= capn) {
-                    atomicOr(overflow, 2);
+            return vx + (int64_t)vy * g.C + (int64_t)vz * g.C * g.R;
+        };
+        if constexpr (G == 1) {
+            ListWriter w(vox, list_buf, base);
+            w.put(last);
+            while (depth > STEP) {
+                if (k >= a.n_steps || (int64_t)s2 >= a.n_coeff) {
+                    atomicOr(overflow, 1);
                     break;
                 }
-                w.put((uint32_t)voxel);
-                cnt++;
-                last = (uint32_t)voxel;
+                u_shifted += STEP;
+                const int64_t voxel = voxel_of(k, s2, depth, u_shifted);
+                if (voxel != (int64_t)last && voxel < g.NV) {
+                    if (cnt >= capn) {
+                        atomicOr(overflow, 2);
+                        break;
+                    }
+                    w.put((uint32_t)voxel);
+                    cnt++;
+                    last = (uint32_t)voxel;
+                }
+                depth -= STEP;
+                s2 -= a.s_step;
+                k++;
             }
-            depth -= STEP;
-            s2 -= a.s_step;
-            k++;
+            w.flush();
+            cnt_out[i] = (uint32_t)cnt;
+        } else {
+            GroupList<G> w{vox + base, capn, 1, last, l};
+            if (l == 0) vox[base] = last;
+            for (bool more = true; more;) {
+                // depth and u_shifted go through every step: a lane's own are sums of as many roundings as there are
+                double d = depth, u = u_shifted;
+#pragma unroll
+                for (int q = 0; q < G; q++) {
+                    u_shifted += STEP;
+                    d = q == l ? depth : d;
+                    u = q == l ? u_shifted : u;
+                    depth -= STEP;
+                }
+                const unsigned c2 = s2 - (unsigned)l * a.s_step;
+                const bool step = d > STEP, ok = k + l < a.n_steps && (int64_t)c2 < a.n_coeff;
+                const uint32_t bad = w.group(__ballot(step && !ok));
+                const bool take = step && (bad & ((2u << l) - 1u)) == 0;
+                const int64_t voxel = take ? voxel_of(k + l, c2, d, u) : 0;
+                const bool room = w.put(take && voxel < g.NV, (uint32_t)voxel);
+                if (l == 0 && (bad || !room)) atomicOr(overflow, bad ? 1 : 2);
+                more = room && !bad && w.group(__ballot(step)) == (1u << G) - 1u;
+                s2 -= (unsigned)G * a.s_step;
+                k += G;
+            }
+            if (l == 0) cnt_out[i] = (uint32_t)w.cnt;
         }
-        w.flush();
-        cnt_out[i] = (uint32_t)cnt;
     }
 }
 
@@ -448,22 +512,25 @@ __global__ void k_mlp_capacity_std(int64_t n, StdArgs a, H10 hp, int64_t* cap)
 }
 
 // One history per lane, grid-stride.  FP64 throughout, with the reference's float powf roundings.
+template <int G>
 __global__ void __launch_bounds__(kBlock) k_mlp_lists_std(int64_t n, StdArgs a, H10 hp,
                                                           const uint32_t* __restrict__ first,
                                                           const int64_t* __restrict__ off,
                                                           uint32_t* __restrict__ cnt_out, uint32_t* __restrict__ vox,
                                                           double* __restrict__ chord, int32_t* overflow)
 {
-    __shared__ uint32_t list_buf[16 * kBlock];
+    __shared__ uint32_t list_buf[G == 1 ? 16 * kBlock : 1];
     const DevGeom& g = a.g;
     const double STEP = a.step, E0 = a.e0, X0 = a.x0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const int l = threadIdx.x & (G - 1);
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x / G;
+    for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; i < n; i += stride) {
         const double x_in = hp.h[0][i], y_in = hp.h[1][i], z_in = hp.h[2][i];
         const double x_out = hp.h[3][i], y_out = hp.h[4][i], z_out = hp.h[5][i];
         const double xy_e0 = hp.h[6][i], xz_entry = hp.h[7][i], xy_x0 = hp.h[8][i], xz_exit = hp.h[9][i];
         // the chord comes from the angles before the +pi turn (DS.cu:8921 precedes :8945)
-        chord[i] = chord_length(g.PI, g.VW, g.VT, STEP, (xy_e0 + xy_x0) / 2.0, (xz_entry + xz_exit) / 2.0);
+        const double L = chord_length(g.PI, g.VW, g.VT, STEP, (xy_e0 + xy_x0) / 2.0, (xz_entry + xz_exit) / 2.0);
+        if (l == 0) chord[i] = L;
         StdFrame f = std_frame(g.PI, x_in, y_in, x_out, y_out, xy_e0, xy_x0);
         const double T0_0 = f.t_in, T0_1 = 0.0, T2_0 = f.t_out, T2_1 = f.xy_exit - f.xy_entry;
         const double V0_0 = z_in, V0_1 = 0.0, V2_0 = z_out, V2_1 = xz_exit - xz_entry;
@@ -477,15 +544,9 @@ __global__ void __launch_bounds__(kBlock) k_mlp_lists_std(int64_t n, StdArgs a, 
         const int64_t base = off[i], capn = off[i + 1] - off[i];
         uint32_t last = first[i];
         int64_t cnt = 1;
-        ListWriter w(vox, list_buf, base);
-        w.put(last);
         double u_1 = STEP;
         int k = 0;
-        while (u_1 < u_2 - STEP) {
-            if (k >= a.max_steps) {
-                atomicOr(overflow, 1);
-                break;
-            }
+        auto voxel_of = [&](double u_1) -> int64_t {
             const double R0_1 = u_1, R1_1 = u_2 - u_1, R1T_2 = u_2 - u_1;
             const double k1 = (double)pct_sqf(E0 * (1 + 0.038 * log((u_1 - u_0) / X0))) / X0;
             const double st1 = k1 * ((double)std_cubef(u_1) * std_poly(a, a.f312, u_1));
@@ -535,21 +596,52 @@ __global__ void __launch_bounds__(kBlock) k_mlp_lists_std(int64_t n, StdArgs a, 
             const int vx = pct_calc_voxel(g.X0, x_1, g.VW);
             const int vy = pct_calc_voxel(g.Y0, y_1, g.VH);
             const int vz = pct_calc_voxel(g.Z0, v_1, g.VT);
-            const int64_t voxel = vx + (int64_t)vy * g.C + (int64_t)vz * g.C * g.R;
-            if (voxel != (int64_t)last && voxel < g.NV) {
-                if (cnt >= capn) {
-                    atomicOr(overflow, 2);
+            return vx + (int64_t)vy * g.C + (int64_t)vz * g.C * g.R;
+        };
+        if constexpr (G == 1) {
+            ListWriter w(vox, list_buf, base);
+            w.put(last);
+            while (u_1 < u_2 - STEP) {
+                if (k >= a.max_steps) {
+                    atomicOr(overflow, 1);
                     break;
                 }
-                w.put((uint32_t)voxel);
-                cnt++;
-                last = (uint32_t)voxel;
+                const int64_t voxel = voxel_of(u_1);
+                if (voxel != (int64_t)last && voxel < g.NV) {
+                    if (cnt >= capn) {
+                        atomicOr(overflow, 2);
+                        break;
+                    }
+                    w.put((uint32_t)voxel);
+                    cnt++;
+                    last = (uint32_t)voxel;
+                }
+                u_1 += STEP;
+                k++;
             }
-            u_1 += STEP;
-            k++;
+            w.flush();
+            cnt_out[i] = (uint32_t)cnt;
+        } else {
+            GroupList<G> w{vox + base, capn, 1, last, l};
+            if (l == 0) vox[base] = last;
+            for (bool more = true; more;) {
+                double u = u_1;
+#pragma unroll
+                for (int q = 0; q < G; q++) {
+                    u = q == l ? u_1 : u;
+                    u_1 += STEP;
+                }
+                const bool step = u < u_2 - STEP;
+                const uint32_t bad = w.group(__ballot(step && k + l >= a.max_steps));
+                const bool take = step && (bad & ((2u << l) - 1u)) == 0;
+                const int64_t voxel = take ? voxel_of(u) : 0;
+                const bool room = w.put(take && voxel < g.NV, (uint32_t)voxel);
+                if (l == 0 && (bad || !room)) atomicOr(overflow, bad ? 1 : 2);
+                more = room && !bad && w.group(__ballot(step)) == (1u << G) - 1u;
+                k += G;
+            }
+            if (l == 0) cnt_out[i] = (uint32_t)w.cnt;
         }
-        w.flush();
-        cnt_out[i] = (uint32_t)cnt;
     }
 }
 
@@ -594,6 +686,15 @@ StdArgs std_args(const pct_params& P, int max_steps)
 }
 
 }  // namespace
+
+// Lanes per history of the list kernels, unless set (PCT_MLP_LANES).  One lane per history leaves most of the chip
+// idle below some 10^5 of them, and the steps of a path do not depend on one another.  Whole list builds with 1 | 4 |
+// 16 lanes, ms: 7.4K histories 0.530 | 0.471 | 0.443, 24K 0.790 | 0.615 | 0.600, 42K 1.266 | 1.049 | 1.088, 141K
+// 1.158 | 1.028 | 1.071, 167K 0.902 | 0.891 | 0.914, 279K 3.780 | 3.776 | 3.996.
+static int mlp_lanes(int64_t histories)
+{
+    return histories <= 1 << 15 ? 16 : histories <= 3 << 16 ? 4 : 1;
+}
 
 // reconstruction_cuts (DS.cu:8296): endpoints on the selected hull, keep histories that hit it
 int pct_stage_endpoints(pct_ctx* ctx)
@@ -739,21 +840,25 @@ int pct_stage_build_lists(pct_ctx* ctx)
         if (m <= 0) return PCT_OK;
         H10 hq;
         for (int k = 0; k < 10; k++) hq.h[k] = ctx->h[k] + h0;
-        const int64_t want = (m + kBlock - 1) / kBlock;
+        const int G = ctx->mlp_lanes ? ctx->mlp_lanes : mlp_lanes(m);
+        const int64_t want = (m * G + kBlock - 1) / kBlock;
         // persistent grid (8 workgroups per CU) when the kernel has the GPU to itself; one lane per history
         // when it shares the GPU with the transposition, so that the two streams' workgroups interleave
         const int per_cu = ctx->mlp_blocks_per_cu >= 0 ? ctx->mlp_blocks_per_cu : (st == ctx->stream ? 8 : 0);
         const int64_t cap_blocks = per_cu > 0 ? (int64_t)dev_cus * per_cu : want;
         const unsigned blocks = (unsigned)(want < cap_blocks ? want : cap_blocks);
-        if (standard)
-            hipLaunchKernelGGL(k_mlp_lists_std, dim3(blocks), dim3(kBlock), 0, st, m, sa, hq, ctx->first_voxel + h0,
+        if (standard) {
+            auto kern = G == 16 ? k_mlp_lists_std<16> : G == 4 ? k_mlp_lists_std<4> : k_mlp_lists_std<1>;
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, st, m, sa, hq, ctx->first_voxel + h0,
                                ctx->list_off + h0, ctx->list_cnt + h0, ctx->list_vox, ctx->chord + h0,
                                ctx->list_overflow);
-        else
-            hipLaunchKernelGGL(k_mlp_lists, dim3(blocks), dim3(kBlock), lds, st, m, a, hq, ctx->first_voxel + h0,
+        } else {
+            auto kern = G == 16 ? k_mlp_lists<16> : G == 4 ? k_mlp_lists<4> : k_mlp_lists<1>;
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), lds, st, m, a, hq, ctx->first_voxel + h0,
                                ctx->T.sin_t, ctx->T.cos_t, ctx->T.scat, ctx->T.p12, ctx->T.p26, ctx->T.p312,
                                ctx->T.step_terms, ctx->list_off + h0, ctx->list_cnt + h0, ctx->list_vox,
                                ctx->chord + h0, ctx->list_overflow);
+        }
         PCT_CHECK_HIP(ctx, hipGetLastError());
         return PCT_OK;
     };
