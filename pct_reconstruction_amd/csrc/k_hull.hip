@@ -34,6 +34,23 @@ __global__ void k_init_counts(DevGeom g, int32_t* counts)
     counts[v] = inside_cylinder(g, c, r);
 }
 
+// The chord of a history: take_3D_step's line (DS.cu:11392).
+__device__ __forceinline__ void chord_line(float xe, float ye, float ze, float xx, float yx, float zx, Walk3& w)
+{
+    w.xs = xe;
+    w.ys = ye;
+    w.zs = ze;
+    w.xm = (xe <= xx) - (xe >= xx);
+    w.ym = (ye <= yx) - (ye >= yx);
+    w.zm = (ze <= zx) - (ze >= zx);
+    w.dy_dx = (double)((yx - ye) / (xx - xe));
+    w.dz_dx = (double)((zx - ze) / (xx - xe));
+    w.dz_dy = (double)((zx - ze) / (yx - ye));
+    w.dx_dy = (double)((xx - xe) / (yx - ye));
+    w.dx_dz = (double)((xx - xe) / (zx - ze));
+    w.dy_dz = (double)((yx - ye) / (zx - ze));
+}
+
 // The entry->exit walk of SC/MSC/SM (take_2D_step_GPU :11346, take_3D_step_GPU :11392).  Visits
 // every voxel from the entry voxel up to, excluding, the exit voxel.  The walk also stops at a
 // negative voxel coordinate or after 4*(C+R+S)+16 steps: there the reference indexes out of bounds
@@ -42,82 +59,57 @@ template <class Visit>
 __device__ void carve_walk(const DevGeom& g, float xe, float ye, float ze, float xx, float yx, float zx, Visit visit)
 {
     const int C = g.C, R = g.R, S = g.S;
-    double x = xe, y = ye, z = ze;
-    int x_move = (xe <= xx) - (xe >= xx);
-    int y_move = (ye <= yx) - (ye >= yx);
-    int z_move = (ze <= zx) - (ze >= zx);
-    int vx = pct_calc_voxel(g.X0, xe, g.VW), vy = pct_calc_voxel(g.Y0, ye, g.VH), vz = pct_calc_voxel(g.Z0, ze, g.VT);
-    int64_t voxel = vx + (int64_t)vy * C + (int64_t)vz * C * R;
-    double x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-    double y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-    double z_to_go = pct_dist(g.Z0, z, PCT_Z_INC, z_move, g.VT, vz);
-    double dy_dx = (double)((yx - ye) / (xx - xe));
-    double dz_dx = (double)((zx - ze) / (xx - xe));
-    double dz_dy = (double)((zx - ze) / (yx - ye));
-    double dx_dy = (double)((xx - xe) / (yx - ye));
-    double dx_dz = (double)((xx - xe) / (zx - ze));
-    double dy_dz = (double)((yx - ye) / (zx - ze));
-    int vxo = pct_calc_voxel(g.X0, xx, g.VW), vyo = pct_calc_voxel(g.Y0, yx, g.VH), vzo = pct_calc_voxel(g.Z0, zx, g.VT);
-    int64_t voxel_out = vxo + (int64_t)vyo * C + (int64_t)vzo * C * R;
-    bool end_walk = (voxel == voxel_out) || (vx >= C) || (vy >= R) || (vz >= S) || vx < 0 || vy < 0 || vz < 0;
-    if (!end_walk) visit(voxel);
+    Walk3 w;
+    chord_line(xe, ye, ze, xx, yx, zx, w);
+    w.ax = w.ay = w.az = w.at = 0;
+    w.vx = pct_calc_voxel(g.X0, xe, g.VW);
+    w.vy = pct_calc_voxel(g.Y0, ye, g.VH);
+    w.vz = pct_calc_voxel(g.Z0, ze, g.VT);
+    const int vxo = pct_calc_voxel(g.X0, xx, g.VW), vyo = pct_calc_voxel(g.Y0, yx, g.VH), vzo = pct_calc_voxel(g.Z0, zx, g.VT);
+    const int64_t voxel_out = vxo + (int64_t)vyo * C + (int64_t)vzo * C * R;
+    auto address = [&] { return w.vx + (int64_t)w.vy * C + (int64_t)w.vz * C * R; };
+    int64_t voxel = address();
+    bool end_walk = voxel == voxel_out || w.vx >= C || w.vy >= R || w.vz >= S || w.vx < 0 || w.vy < 0 || w.vz < 0;
     const int cap = 4 * (C + R + S) + 16;
     int steps = 0;
-    while (!end_walk) {
-        if (z_move != 0) {
-            double x_ext = fabs(dz_dx) * x_to_go;
-            double y_ext = fabs(dz_dy) * y_to_go;
-            if ((z_to_go <= x_ext) && (z_to_go <= y_ext)) {
-                vz -= z_move;
-                z = pct_edge(g.Z0, vz, g.VT, PCT_Z_INC, z_move);
-                x = pct_corr(dx_dz, z, ze, xe);
-                y = pct_corr(dy_dz, z, ze, ye);
-                x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-                z_to_go = g.VT;
-            } else if (x_ext <= y_ext) {
-                vx += x_move;
-                x = pct_edge(g.X0, vx, g.VW, PCT_X_INC, x_move);
-                y = pct_corr(dy_dx, x, xe, ye);
-                z = pct_corr(dz_dx, x, xe, ze);
-                x_to_go = g.VW;
-                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-                z_to_go = pct_dist(g.Z0, z, PCT_Z_INC, z_move, g.VT, vz);
-            } else {
-                vy -= y_move;
-                y = pct_edge(g.Y0, vy, g.VH, PCT_Y_INC, y_move);
-                x = pct_corr(dx_dy, y, ye, xe);
-                z = pct_corr(dz_dy, y, ye, ze);
-                x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-                y_to_go = g.VH;
-                z_to_go = pct_dist(g.Z0, z, PCT_Z_INC, z_move, g.VT, vz);
-            }
-            if (x_to_go == 0) { x_to_go = g.VW; vx += x_move; }
-            if (y_to_go == 0) { y_to_go = g.VH; vy -= y_move; }
-            if (z_to_go == 0) { z_to_go = g.VT; vz -= z_move; }
-        } else {
-            double y_ext = fabs(dx_dy) * y_to_go;
-            if (x_to_go <= y_ext) {
-                vx += x_move;
-                x = pct_edge(g.X0, vx, g.VW, PCT_X_INC, x_move);
-                y = pct_corr(dy_dx, x, xe, ye);
-                x_to_go = g.VW;
-                y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, y_move, g.VH, vy);
-            } else {
-                vy -= y_move;
-                y = pct_edge(g.Y0, vy, g.VH, PCT_Y_INC, y_move);
-                x = pct_corr(dx_dy, y, ye, xe);
-                x_to_go = pct_dist(g.X0, x, PCT_X_INC, x_move, g.VW, vx);
-                y_to_go = g.VH;
-            }
-            if (x_to_go == 0) { x_to_go = g.VW; vx += x_move; }
-            if (y_to_go == 0) { y_to_go = g.VH; vy -= y_move; }
+    auto stepped = [&] {
+        voxel = address();
+        end_walk = voxel == voxel_out || w.vx >= C || w.vy >= R || w.vz >= S || w.vx < 0 || w.vy < 0 || ++steps > cap;
+    };
+    if (w.zm != 0) {
+        w.begin(g);
+        while (!end_walk) {
+            visit(voxel);
+            int full;
+            bool clamped;
+            w.step(g, &full, &clamped);
+            stepped();
         }
-        vz = vz > 0 ? vz : 0;
-        voxel = vx + (int64_t)vy * C + (int64_t)vz * C * R;
-        end_walk = (voxel == voxel_out) || (vx >= C) || (vy >= R) || (vz >= S);
-        if (vx < 0 || vy < 0 || ++steps > cap) end_walk = true;
-        if (!end_walk) visit(voxel);
+        return;
+    }
+    double x = xe, y = ye;
+    double x_to_go = pct_dist(g.X0, x, PCT_X_INC, w.xm, g.VW, w.vx);
+    double y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, w.ym, g.VH, w.vy);
+    while (!end_walk) {
+        visit(voxel);
+        const double y_ext = fabs(w.dx_dy) * y_to_go;
+        if (x_to_go <= y_ext) {
+            w.vx += w.xm;
+            x = pct_edge(g.X0, w.vx, g.VW, PCT_X_INC, w.xm);
+            y = pct_corr(w.dy_dx, x, xe, ye);
+            x_to_go = g.VW;
+            y_to_go = pct_dist(g.Y0, y, PCT_Y_INC, w.ym, g.VH, w.vy);
+        } else {
+            w.vy -= w.ym;
+            y = pct_edge(g.Y0, w.vy, g.VH, PCT_Y_INC, w.ym);
+            x = pct_corr(w.dx_dy, y, ye, xe);
+            x_to_go = pct_dist(g.X0, x, PCT_X_INC, w.xm, g.VW, w.vx);
+            y_to_go = g.VH;
+        }
+        if (x_to_go == 0) { x_to_go = g.VW; w.vx += w.xm; }
+        if (y_to_go == 0) { y_to_go = g.VH; w.vy -= w.ym; }
+        w.vz = w.vz > 0 ? w.vz : 0;
+        stepped();
     }
 }
 
@@ -243,22 +235,6 @@ __device__ __forceinline__ uint32_t carve_tile(int vx, int vy, int vz, int ntx, 
     return ((uint32_t)(vz >> 1) * nty + (uint32_t)(vy >> 6)) * ntx + (uint32_t)(vx >> 6);
 }
 
-__device__ __forceinline__ void chord_line(const CarveRec& r, Walk3& w)
-{
-    w.xs = r.xe;
-    w.ys = r.ye;
-    w.zs = r.ze;
-    w.xm = (r.xe <= r.xx) - (r.xe >= r.xx);
-    w.ym = (r.ye <= r.yx) - (r.ye >= r.yx);
-    w.zm = (r.ze <= r.zx) - (r.ze >= r.zx);
-    w.dy_dx = (double)((r.yx - r.ye) / (r.xx - r.xe));
-    w.dz_dx = (double)((r.zx - r.ze) / (r.xx - r.xe));
-    w.dz_dy = (double)((r.zx - r.ze) / (r.yx - r.ye));
-    w.dx_dy = (double)((r.xx - r.xe) / (r.yx - r.ye));
-    w.dx_dz = (double)((r.xx - r.xe) / (r.zx - r.ze));
-    w.dy_dz = (double)((r.yx - r.ye) / (r.zx - r.ze));
-}
-
 // The histories of a batch in visiting order, and how many tile entries each may have: one more than the tile steps
 // between its first and last voxel, and one for a start on a tile's far edge; none when no method takes it.  cap[n] is
 // 0: the scan's total.
@@ -310,7 +286,7 @@ __global__ void __launch_bounds__(256) k_carve_cut(int64_t n, DevGeom g, const C
     };
     if (r.inc) {
         Walk3 w;
-        chord_line(r, w);
+        chord_line(r.xe, r.ye, r.ze, r.xx, r.yx, r.zx, w);
         if (w.zm == 0) {
             carve_walk(g, r.xe, r.ye, r.ze, r.xx, r.yx, r.zx, count);
         } else {
@@ -444,7 +420,7 @@ __global__ void __launch_bounds__(kCarveBlock) k_carve_tiles(DevGeom g, const Ca
         const CarveRec r = recs[(uint32_t)v];
         const uint32_t s = (uint32_t)(v >> 32);
         Walk3 w;
-        chord_line(r, w);
+        chord_line(r.xe, r.ye, r.ze, r.xx, r.yx, r.zx, w);
         w.vx = bx + (int)(s & 63u);
         w.vy = by + (int)((s >> 6) & 63u);
         w.vz = bz + (int)((s >> 12) & 1u);
