@@ -620,10 +620,14 @@ def main() -> int:
         return {"avg_launch_ms": ms, "bytes_per_launch": nbytes, "GBs": nbytes / (ms * 1e-3) / 1e9,
                 "launches_per_step": launches_per_step, "ms_per_step": ms * launches_per_step}
 
+    tiles = bool(m["drop_plan"]["tiles"])
     kernels = {
         "drop_rows": kern(prof["rows_ms"], rows_bytes, iters * nb),
         "drop_cols": kern(prof["cols_ms"], cols_bytes, iters * nb),
     }
+    if tiles:  # k_tile_rows and k_tile_pass share the entries' work otherwise: only the block's bytes are counted
+        for k in ("drop_rows", "drop_cols"):
+            del kernels[k]["bytes_per_launch"], kernels[k]["GBs"]
     if segs:  # one MLP launch per segment and iteration; the last segment's launch time
         ns = max(segs["count"], 1)
         kernels["mlp_lists"] = kern(mlp_ms, mlp_bytes / ns, iters * ns)
@@ -633,7 +637,8 @@ def main() -> int:
         kernels["mlp_lists"] = kern(mlp_ms, mlp_bytes, 1)
         kernels["list_transpose_ms_per_step"] = max(m["stage_ms"]["mlp_build_lists"] - mlp_ms, 0.0)
     # The dominant work is the DROP block update, which the reference performs as
-    # calculate_x_update_GPU + image_update_GPU and this build as the pair k_drop_rows + k_drop_cols.
+    # calculate_x_update_GPU + image_update_GPU and this library as the pair k_tile_rows + k_tile_pass, or, with
+    # sorted lists, k_drop_rows + k_drop_cols.
     # Its algorithmic bytes per proton-iteration are B_alg = 18 n + 12 (list entry 6 B incl. chord,
     # x gather 4 B, x_update read-modify-write 8 B per voxel; 8 B header + 4 B WEPL per proton),
     # priced per block and divided by the block's average rows + cols duration.
@@ -652,7 +657,8 @@ def main() -> int:
                 traffic_src = f"stored: {tfile.relative_to(ROOT)} (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE)"
         except (OSError, ValueError):
             traffic = None
-    roofline = {"bound": "hbm", "kernel": "drop_block (k_drop_rows + k_drop_cols per DROP block)",
+    roofline = {"bound": "hbm", "kernel": ("drop_block (k_tile_rows + k_tile_pass per DROP block)" if tiles else
+                                          "drop_block (k_drop_rows + k_drop_cols per DROP block)"),
                 "achieved": block_bytes / (block_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": block_bytes / (block_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": traffic,
                 "traffic_source": traffic_src, "bytes_per_launch": block_bytes, "avg_launch_ms": block_ms}

@@ -1,4 +1,6 @@
-// k_drop2.hip — stage (e): atomic-free DROP over per-block transposed path lists.
+// k_drop2.hip — stage (e): atomic-free DROP over per-block transposed path lists.  Large plans with the default
+// flags take k_drop_tiles.hip instead (pct_drop_prepare); these kernels run the smaller and sparser ones and every
+// other launch shape, where the tiles' own costs outweigh the gathers that they save.
 //
 // DROP (DROP_full_tx_iteration, DS.cu:9537-9589) updates every voxel of a block by the mean of the
 // updates of the block's histories through it:
