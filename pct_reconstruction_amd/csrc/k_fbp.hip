@@ -68,82 +68,95 @@ struct BPArgs {
     int quirk_decode;
 };
 
-// backprojection_GPU2, DS.cu:6340-6479
-__global__ void k_backproject(BPArgs a, const float* __restrict__ sf, const double* __restrict__ cs, float* image)
+// backprojection_GPU2, DS.cu:6340-6479.  Bound by its FP64 arithmetic: five divisions for a voxel and an angle, three
+// of which, with everything else that leads to the t bin, do not depend on z.  A lane takes ZC voxels of one column and
+// forms those once.  6.3M voxels and 90 angles: 1.35 ms with ZC = 8, 2.15 with 1.
+template <int ZC>
+__global__ void k_backproject(BPArgs a, const float* __restrict__ sf, const double* __restrict__ cs,
+                              unsigned per_chunk, float* __restrict__ image)
 {
-    int64_t voxel = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (voxel >= a.NV) return;
-    int vx, vy, vz;
-    const int64_t CR = (int64_t)a.C * a.R;
-    if (a.quirk_decode) {  // voxel_2_3D_voxels_GPU, DS.cu:11124-11134 ('>' comparisons)
-        int64_t rem = voxel, z = 0, y = 0;
-        if (rem - CR > 0) {
-            z = (rem - 1) / CR;
-            rem -= z * CR;
-        }
+    const int64_t CR = (int64_t)a.C * a.R, column = (int64_t)(blockIdx.x % per_chunk) * blockDim.x + threadIdx.x;
+    const int z0 = (int)(blockIdx.x / per_chunk) * ZC;
+    int vx, vy, n = a.S - z0 < ZC ? a.S - z0 : ZC;
+    if (a.quirk_decode) {  // voxel_2_3D_voxels_GPU, DS.cu:11124-11134 ('>' comparisons): columns 1..CR, and voxel 0
+        if (column > CR) return;
+        int64_t rem = column, y = 0;
         if (rem - a.C > 0) {
             y = (rem - 1) / a.C;
             rem -= y * a.C;
         }
         vx = (int)rem;
         vy = (int)y;
-        vz = (int)z;
+        if (column == 0) n = z0 == 0 ? 1 : 0;
     } else {
-        vz = (int)(voxel / CR);
-        vy = (int)((voxel / a.C) % a.R);
-        vx = (int)(voxel % a.C);
+        if (column >= CR) return;
+        vy = (int)(column / a.C);
+        vx = (int)(column % a.C);
     }
+    if (column + (int64_t)(z0 + n - 1) * CR >= a.NV) n--;  // the last column's last voxel is past the image
+    if (n <= 0) return;
+    float* out = image + column + (int64_t)z0 * CR;
     double x = 1 * (vx - (a.C - 1) / 2.0) * a.VW;
     double y = -1 * (vy - (a.R - 1) / 2.0) * a.VH;
-    double z = -1 * (vz - (a.S - 1) / 2.0) * a.VT;
     if ((x * x + y * y) > (a.Rc * a.Rc)) {
-        image[voxel] = a.rsp_air;
+        for (int k = 0; k < n; k++) out[k * CR] = a.rsp_air;
         return;
     }
     const int T = a.T, V = a.V, A = a.A;
-    float acc = 0.0f;
+    float acc[ZC];
+#pragma unroll
+    for (int k = 0; k < ZC; k++) acc[k] = 0.0f;
     for (int ab = 0; ab < A; ab++) {
         const double c = cs[ab], sn = cs[A + ab];
         double u = x * c + y * sn;
         double t = y * c - x * sn;
-        double v = z;
         double dnt = (t - u * (t / (a.SR + u))) / a.t_bin_size + T / 2.0;
         int t_bin = (int)floor(dnt);
         double eta = dnt - t_bin;
-        double dnv = (v - u * (v / (a.SR + u))) / a.v_bin_size + V / 2.0;
-        int v_bin = (int)floor(dnv);
-        double eps = dnv - v_bin;
         double scale = (double)pct_sqf(a.SR / (a.SR + u));
-        int64_t b11 = ((int64_t)v_bin * A + ab) * T + t_bin;
-        int64_t b12 = b11 + 1, b21 = b11 + (int64_t)A * T, b22 = b21 + 1;
-        float xterm = 0.0f;
-        if (t_bin > -1 && t_bin < T - 1) {
-            if (v_bin > -1 && v_bin < V - 1)
-                xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps) + (double)sf[b12] * eta * (1 - eps) +
-                                (double)sf[b21] * (1 - eta) * eps + (double)sf[b22] * eta * eps);
-            else if (v_bin == -1)
-                xterm = (float)((double)sf[b21] * (1 - eta) * eps + (double)sf[b22] * eta * eps);
-            else if (v_bin == V - 1)
-                xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps) + (double)sf[b12] * eta * (1 - eps));
-        } else if (t_bin == -1) {
-            if (v_bin > -1 && v_bin < V - 1)
-                xterm = (float)((double)sf[b12] * eta * (1 - eps) + (double)sf[b22] * eta * eps);
-            else if (v_bin == -1)
-                xterm = (float)((double)sf[b22] * eta * eps);
-            else if (v_bin == V - 1)
-                xterm = (float)((double)sf[b12] * eta * (1 - eps));
-        } else if (t_bin == T - 1) {
-            if (v_bin > -1 && v_bin < V - 1)
-                xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps) + (double)sf[b21] * (1 - eta) * eps);
-            else if (v_bin == -1)
-                xterm = (float)((double)sf[b21] * (1 - eta) * eps);
-            else if (v_bin == V - 1)
-                xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps));
+#pragma unroll
+        for (int k = 0; k < ZC; k++) {
+            if (k >= n) break;
+            const double v = -1 * (z0 + k - (a.S - 1) / 2.0) * a.VT;
+            double dnv = (v - u * (v / (a.SR + u))) / a.v_bin_size + V / 2.0;
+            int v_bin = (int)floor(dnv);
+            double eps = dnv - v_bin;
+            int64_t b11 = ((int64_t)v_bin * A + ab) * T + t_bin;
+            int64_t b12 = b11 + 1, b21 = b11 + (int64_t)A * T, b22 = b21 + 1;
+            float xterm = 0.0f;
+            if (t_bin > -1 && t_bin < T - 1) {
+                if (v_bin > -1 && v_bin < V - 1)
+                    xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps) + (double)sf[b12] * eta * (1 - eps) +
+                                    (double)sf[b21] * (1 - eta) * eps + (double)sf[b22] * eta * eps);
+                else if (v_bin == -1)
+                    xterm = (float)((double)sf[b21] * (1 - eta) * eps + (double)sf[b22] * eta * eps);
+                else if (v_bin == V - 1)
+                    xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps) + (double)sf[b12] * eta * (1 - eps));
+            } else if (t_bin == -1) {
+                if (v_bin > -1 && v_bin < V - 1)
+                    xterm = (float)((double)sf[b12] * eta * (1 - eps) + (double)sf[b22] * eta * eps);
+                else if (v_bin == -1)
+                    xterm = (float)((double)sf[b22] * eta * eps);
+                else if (v_bin == V - 1)
+                    xterm = (float)((double)sf[b12] * eta * (1 - eps));
+            } else if (t_bin == T - 1) {
+                if (v_bin > -1 && v_bin < V - 1)
+                    xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps) + (double)sf[b21] * (1 - eta) * eps);
+                else if (v_bin == -1)
+                    xterm = (float)((double)sf[b21] * (1 - eta) * eps);
+                else if (v_bin == V - 1)
+                    xterm = (float)((double)sf[b11] * (1 - eta) * (1 - eps));
+            }
+            acc[k] += (float)((double)xterm * a.delta * scale);
         }
-        acc += (float)((double)xterm * a.delta * scale);
     }
-    image[voxel] = acc;
+#pragma unroll
+    for (int k = 0; k < ZC; k++)
+        if (k < n) out[k * CR] = acc[k];
 }
+
+// Voxels of a column per lane: 8 while that leaves lanes to fill the chip (2^18), else 1.
+constexpr int64_t kColumnLanes = 1 << 18;
 
 }  // namespace
 
@@ -195,8 +208,14 @@ int pct_stage_fbp(pct_ctx* ctx)
     a.delta = delta;
     a.rsp_air = (float)P.rsp_air;
     a.quirk_decode = P.quirk_voxel_decode;
-    hipLaunchKernelGGL(k_backproject, dim3(grid_for(P.num_voxels)), dim3(kBlock), 0, s, a, ctx->sino_filtered, d_cs,
-                       ctx->fbp);
+    const int64_t columns = (int64_t)P.columns * P.rows, chunks8 = (P.slices + 7) / 8;
+    const unsigned per_chunk = grid_for(columns + 1);  // workgroups
+    const bool eight = columns * chunks8 >= kColumnLanes;
+    const unsigned grid = grid_for((int64_t)per_chunk * kBlock * (eight ? chunks8 : P.slices));
+    if (eight)
+        hipLaunchKernelGGL(k_backproject<8>, dim3(grid), dim3(kBlock), 0, s, a, ctx->sino_filtered, d_cs, per_chunk, ctx->fbp);
+    else
+        hipLaunchKernelGGL(k_backproject<1>, dim3(grid), dim3(kBlock), 0, s, a, ctx->sino_filtered, d_cs, per_chunk, ctx->fbp);
     PCT_CHECK_HIP(ctx, hipGetLastError());
     PCT_TRY(pct_median_filter_fbp(ctx));  // FBP(), DS.cu:6150-6166 (x0 only)
     if (P.hull_type == PCT_HULL_FBP) PCT_TRY(pct_fbp_hull(ctx));
