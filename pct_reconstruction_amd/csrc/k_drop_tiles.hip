@@ -4,7 +4,8 @@
 // gathers bounds them.  Here a DROP block's lists are cut, when they are built, into segments: runs of
 // consecutive entries inside one tile of 16 x 16 x 2 voxels (512 floats, 2 KB).  A segment holds about 11
 // entries, and 220 segments of a block pass through a tile (head, blocks of 60000), so a workgroup that owns a
-// tile reads its 512 voxels once and each segment's update once, and every gather per entry is an LDS read.  Per block b two kernels run:
+// tile reads its 512 voxels once and each segment's update once, and every gather per entry is an LDS read.  Per
+// block b two kernels run:
 //   k_tile_rows  8 lanes per history: adds the partial row sums of its segments and forms u_i
 //                (DS.cu:9321-9380), in visiting order;
 //   k_tile_pass  a workgroup per tile: the column sums of block b (u of the tile's segments in LDS, one
@@ -12,7 +13,8 @@
 //                LDS, the partial row sums of block b + 1.  A tile is written by its own workgroup only.
 // The sums are those of k_drop2.hip to the bit: column sums add the same updates in the same order, and a
 // row's partial sums are used only where no sum of its terms can round in any order (order_free, with the
-// bounds taken over the whole tile); every other row is summed in list order from memory.
+// bounds of the whole tile, or of the segment's own values where the tile's span many powers of two: kWide);
+// every other row is summed in list order from memory.
 //
 // Layout of one (block, tile), built by k_tile_fill:
 //   segments in visiting order (neighbouring paths next to each other, so the loads of u and the reads of
