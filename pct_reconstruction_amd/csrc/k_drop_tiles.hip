@@ -171,7 +171,8 @@ __global__ void k_tile_hist_keys(int64_t h0, int64_t n, int64_t BS, int64_t rb0,
 
 // Cuts every history's list into segments (consecutive entries of one tile, steps of at most 127 slots), 16 lanes per history, kRound entries at a time, the histories in
 // visiting order.  EMIT false: the number of segments (0 when it is not processed or shorter than
-// MIN_MLP_LENGTH).  EMIT true: its row descriptor, and per segment the key (block in group, tile) and its record.
+// MIN_MLP_LENGTH).  EMIT true: its row descriptor, and per segment the key (block in group, tile) and its record;
+// without any segment only the descriptors, and the arrays of the segments may be null.
 struct CutArgs {
     int64_t h0, n, BS, rb0, slot0;  // slot0: the group's first list slot
     TileGeom g;
@@ -980,7 +981,10 @@ int build_group(pct_ctx* ctx, TilePlan& T, TileGroup& G, const CutArgs& ca, int 
     if (Q > (1u << 30)) return PCT_OK;
     G.segs = Q;
     G.n_runs = 0;
-    if (Q == 0) {
+    if (Q == 0) {  // nothing to sort, but every history has its row, without segments
+        hipLaunchKernelGGL(k_tile_cut<true>, dim3(cg), dim3(kBlock), 0, s, a, (uint32_t*)nullptr, W.q0, T.rows,
+                           (uint32_t*)nullptr, (uint32_t*)nullptr, (SegRec*)nullptr);
+        PCT_CHECK_HIP(ctx, hipGetLastError());
         *fits = true;
         return PCT_OK;
     }
