@@ -590,9 +590,10 @@ const char* pct_metrics_json(pct_ctx* ctx)
     (void)hipMemGetInfo(&mem_free, &mem_total);
     const bool segmented = ctx->stage >= ST_LISTS && pct_segment_histories(ctx) > 0;
     std::snprintf(buf, sizeof(buf),
-                  ", \"list_entries\": %lld, \"list_slots\": %lld, \"list_capacity\": %lld, \"device_bytes_used\": %lld",
+                  ", \"list_entries\": %lld, \"list_slots\": %lld, \"list_capacity\": %lld, \"device_bytes_used\": %lld"
+                  ", \"device_allocations\": %lld",
                   (long long)(segmented ? ctx->seg.entries : ctx->list_entries), (long long)ctx->list_slots,
-                  (long long)ctx->list_cap, (long long)(mem_total - mem_free));
+                  (long long)ctx->list_cap, (long long)(mem_total - mem_free), (long long)ctx->allocations);
     s += buf;
     if (segmented) {
         std::snprintf(buf, sizeof(buf),

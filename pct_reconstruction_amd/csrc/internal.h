@@ -183,6 +183,8 @@ struct DropPlan {
     int64_t cap_bk = 0;
     int64_t groups_bucketed = 0, groups_sorted = 0;  // groups transposed by each path in the last build
     TilePlan tile;               // tile.ready: the plan is over image tiles and the arrays above are unused
+    // Between segments, of which some take one plan and some the other, both plans' arrays stay: those of the other one
+    enum { IDLE_NONE, IDLE_LISTS, IDLE_TILES } idle = IDLE_NONE;
     int flags = -1;              // PCT_DROP_* flags the plan was built with
     bool desc_all = false;       // desc holds a descriptor for every reconstruction history
     bool ready = false;
@@ -249,6 +251,7 @@ struct pct_ctx {
     uint32_t* u32_d = nullptr;
     void* cub_tmp = nullptr;
     uint8_t* scratch[6] = {};      // by ScratchSlot
+    int64_t allocations = 0;       // device allocations made for the context (metrics)
     void* read_h = nullptr;        // pinned, kReadBytes: where small results land (pct_read)
     double* angle_cs = nullptr;    // cos and sin of the angle bins, as the binning and as the FBP form them
     size_t cub_tmp_bytes = 0;
@@ -336,6 +339,8 @@ struct pct_ctx {
 };
 
 // allocation helpers
+// Frees what the context keeps only to use it again (no memory); true if there was any.
+bool pct_give_back(pct_ctx* ctx);
 // A buffer that is there already and holds `count` elements, with at most a quarter and 64 KB to spare, stays: a
 // context that runs its stages again asks for the same sizes, and a free and an allocation took 10 to 60 us each
 // time, 33 times in a reconstruction.
@@ -354,6 +359,11 @@ int pct_alloc(pct_ctx* ctx, T** p, size_t count)
         *p = nullptr;
     }
     hipError_t e = hipMalloc((void**)p, count * sizeof(T));
+    ctx->allocations++;
+    if (e != hipSuccess && pct_give_back(ctx)) {
+        (void)hipGetLastError();
+        e = hipMalloc((void**)p, count * sizeof(T));
+    }
     if (e != hipSuccess) {
         ctx->err = std::string("hipMalloc(") + std::to_string(count * sizeof(T)) + " B): " + hipGetErrorString(e);
         *p = nullptr;

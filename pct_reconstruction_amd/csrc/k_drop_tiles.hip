@@ -1301,16 +1301,12 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
         *lists_built = true;
     }
     if (!fits) {
-        pct_tile_plan_free(&T);
         if (density > 0.0) T.too_dense = density;  // lists this dense go to the sort at once from here on
         return PCT_OK;
     }
     int64_t segs = 0;
     for (int64_t gi = 0; gi < ng; gi++) segs += T.groups[gi].segs;
-    if (segs == 0) {  // no history is long enough to update a voxel
-        pct_tile_plan_free(&T);
-        return PCT_OK;
-    }
+    if (segs == 0) return PCT_OK;  // no history is long enough to update a voxel
     // the tiles any block touches, and the descriptor of every (block, used tile)
     std::vector<uint8_t> used(g.nt);
     std::vector<BlockTotals> totals(n_raw);
@@ -1324,7 +1320,6 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
         if (used[k]) index_of[k] = (uint32_t)U++;
     T.n_used = U;
     if (nb * U > kMaxTable) {
-        pct_tile_plan_free(&T);
         if (density > 0.0) T.too_dense = density;
         return PCT_OK;
     }
