@@ -211,9 +211,10 @@ int pct_drop_iterate(pct_ctx* ctx, int iterations);
 int pct_run_pipeline(pct_ctx* ctx);
 /* Reset the iterate x to the initial iterate x0 (on the device). */
 int pct_reset_iterate(pct_ctx* ctx);
-/* Launch shape of the DROP kernels: lanes per history in the row kernel (4, 8, 16, 32, 64), voxels
- * per lane in the column kernel (1, 2, 4, 8) and enum pct_drop_flags (a change of flags rebuilds
- * the transposed lists at the next DROP call).  Results do not depend on any of them. */
+/* Launch shape of the DROP kernels: lanes per history in the row kernel (0: by the blocks' sizes, the
+ * default; or 4, 8, 16, 32, 64), voxels per lane in the column kernel (1, 2, 4, 8) and enum
+ * pct_drop_flags (a change of flags rebuilds the transposed lists at the next DROP call).  Results do
+ * not depend on any of them. */
 int pct_set_launch(pct_ctx* ctx, int drop_row_lanes, int drop_col_voxels, int drop_flags);
 /* Run `iterations` DROP iterations with a HIP event pair around every kernel launch and report the
  * average duration of one block's row kernel (per-history updates) and column kernel (per-voxel
