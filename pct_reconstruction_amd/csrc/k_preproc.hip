@@ -279,15 +279,27 @@ __global__ void k_bin_gather(int64_t n, const uint32_t* __restrict__ perm, const
 // (:5937-5971), each over the bin's histories in ascending history order, read from the bin-ordered
 // inputs of k_bin_gather.  The inputs of a wavefront's 64 bins are one contiguous range: it goes to LDS by whole
 // lines, kStatChunk entries at a time, once for the three passes where it fits (from memory a lane used 4 or 8 bytes
-// of each line that it read: 2.2 ms for 16M histories in 1.3M bins, now 0.35).  `failed` is zero on entry.
+// of each line that it read: 2.2 ms for 16M histories in 1.3M bins, now 0.35).  A chunk of well-filled bins keeps few
+// lanes busy, though: a wavefront with more than `most` entries lets every lane read its bin from memory.
+// `failed` is zero on entry.
 constexpr int kStatChunk = 1024;
+struct BinInputs {
+    const uint8_t* ir;
+    const float* w;
+    const double *ut, *uv;
+    Words uv_words;  // where uv is null
+    __device__ __forceinline__ double at_uv(int j) const
+    {
+        return uv ? uv[j] : __hiloint2double((int)uv_words.hi[j], (int)uv_words.lo[j]);
+    }
+};
 __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restrict__ off,
                                                   const uint32_t* __restrict__ perm, const uint8_t* __restrict__ g_ir,
                                                   const float* __restrict__ g_w, const double* __restrict__ g_ut,
                                                   Words g_uv, int32_t* counts_pre, float* m_w,
                                                   float* m_ut, float* m_uv, float* s_w, float* s_ut, float* s_uv,
                                                   int32_t* counts_post, float* sinogram, uint8_t* failed, float k,
-                                                  int quirk_a1)
+                                                  int quirk_a1, int most)
 {
     __shared__ double l_ut[kStatChunk], l_uv[kStatChunk];
     __shared__ float l_w[kStatChunk];
@@ -295,8 +307,14 @@ __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restr
     const int b0 = blockIdx.x * 64, b = b0 + (int)threadIdx.x;
     const int32_t lo = off[b0], hi = off[b0 + 64 < NB ? b0 + 64 : NB];
     const int32_t beg = b < NB ? off[b] : hi, end = b < NB ? off[b + 1] : hi;
-    // f(entry, its place in LDS) over the bin's entries
+    const BinInputs staged{l_ir, l_w, l_ut, l_uv, {}}, in_memory{g_ir, g_w, g_ut, nullptr, g_uv};
+    const bool direct = hi - lo > most;
+    // f(entry, inputs, its place there) over the bin's entries
     auto each = [&](bool first, auto f) {
+        if (direct) {
+            for (int32_t j = beg; j < end; j++) f(j, in_memory, j);
+            return;
+        }
         for (int64_t c0 = lo; c0 < hi; c0 += kStatChunk) {
             if (first || hi - lo > kStatChunk) {
                 __syncthreads();
@@ -311,17 +329,17 @@ __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restr
                 __syncthreads();
             }
             const int64_t last = end < c0 + kStatChunk ? end : c0 + kStatChunk;
-            for (int64_t j = beg > c0 ? beg : c0; j < last; j++) f((int32_t)j, (int)(j - c0));
+            for (int64_t j = beg > c0 ? beg : c0; j < last; j++) f((int32_t)j, staged, (int)(j - c0));
         }
     };
     int cnt = 0;
     float sw = 0.0f, su = 0.0f, sv = 0.0f;
-    each(true, [&](int32_t, int j) {
-        if (!l_ir[j]) return;
+    each(true, [&](int32_t, const BinInputs& in, int j) {
+        if (!in.ir[j]) return;
         cnt += 1;
-        sw += l_w[j];
-        su += (float)l_ut[j];
-        sv += (float)l_uv[j];
+        sw += in.w[j];
+        su += (float)in.ut[j];
+        sv += (float)in.at_uv(j);
     });
     if (cnt > 0) {
         sw /= cnt;
@@ -329,11 +347,11 @@ __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restr
         sv /= cnt;
     }
     float qw = 0.0f, qu = 0.0f, qv = 0.0f;
-    each(false, [&](int32_t, int j) {
-        if (!quirk_a1 && !l_ir[j]) return;
-        double d_w = (double)(l_w[j] - sw);
-        double d_ut = l_ut[j] - su;
-        double d_uv = l_uv[j] - sv;
+    each(false, [&](int32_t, const BinInputs& in, int j) {
+        if (!quirk_a1 && !in.ir[j]) return;
+        double d_w = (double)(in.w[j] - sw);
+        double d_ut = in.ut[j] - su;
+        double d_uv = in.at_uv(j) - sv;
         qw += pct_sqf(d_w);
         qu += pct_sqf(d_ut);
         qv += pct_sqf(d_uv);
@@ -345,14 +363,14 @@ __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restr
     }
     int cpost = 0;
     float sino = 0.0f;
-    each(false, [&](int32_t at, int j) {
-        if (!quirk_a1 && !l_ir[j]) {
+    each(false, [&](int32_t at, const BinInputs& in, int j) {
+        if (!quirk_a1 && !in.ir[j]) {
             failed[perm[at]] = 1;
             return;
         }
-        const float w = l_w[j];
-        int pass_ut = fabs(l_ut[j] - su) < (double)(k * qu);
-        int pass_uv = fabs(l_uv[j] - sv) < (double)(k * qv);
+        const float w = in.w[j];
+        int pass_ut = fabs(in.ut[j] - su) < (double)(k * qu);
+        int pass_uv = fabs(in.at_uv(j) - sv) < (double)(k * qv);
         int pass_w = fabsf(sw - w) <= k * qw;
         if (!pass_ut || !pass_uv || !pass_w) {
             failed[perm[at]] = 1;
@@ -372,6 +390,12 @@ __global__ void __launch_bounds__(64) k_bin_stats(int NB, const int32_t* __restr
     counts_post[b] = cpost;
     sinogram[b] = sino;
 }
+
+// Entries of 64 bins up to which they go through LDS.  Wavefronts that fill the chip are bound by memory and gain from
+// whole lines longer than few ones, which wait for the busiest.  Cuts with LDS | from memory, ms: 16M histories, 71 in a
+// bin 2.93 | 4.69, 117 (2139 wavefronts) 3.49 | 4.26, 233 5.99 | 3.49, 462 12.6 | 3.9; 2M, 22 in a bin (1426 wavefronts)
+// 0.35 | 0.44, 58 (541) 0.53 | 0.46, 115 1.13 | 0.57; 0.3M, 74 (63 wavefronts) 0.66 | 0.23.
+int stat_staged(int bins) { return bins >= 64 * 2048 ? 8192 : 2048; }
 
 }  // namespace
 
@@ -612,7 +636,7 @@ int pct_stage_stats_and_cuts(pct_ctx* ctx)
     hipLaunchKernelGGL(k_bin_stats, dim3(pct_grid_for(NB, 64)), dim3(64), 0, s, NB, ctx->bin_off, perm, g_ir, g_w,
                        g_ut, g_uv, ctx->counts_pre, ctx->mean[0], ctx->mean[1], ctx->mean[2], ctx->stddev[0],
                        ctx->stddev[1], ctx->stddev[2], ctx->counts_post, ctx->sinogram, failed,
-                       (float)P.sigmas_2_keep, P.quirk_a1_bin0);
+                       (float)P.sigmas_2_keep, P.quirk_a1_bin0, stat_staged(NB));
     PCT_CHECK_HIP(ctx, hipGetLastError());
     // keep the histories that passed (DS.cu:5892-5911)
     int64_t kept = 0;
