@@ -378,7 +378,7 @@ void pct_free(T** p)
     *p = nullptr;
 }
 // Scratch of one stage, kept by the context for its next run; every use is on the context's stream, in order.
-enum ScratchSlot { SCR_THRESHOLD, SCR_HULL_BITS, SCR_BLOCK_PROC, SCR_BLOCK_ENTRIES, SCR_BLOCK_SLOTS, SCR_TILE_MARK };
+enum ScratchSlot { SCR_THRESHOLD, SCR_HULL_BITS, SCR_BLOCK_PROC, SCR_BLOCK_ENTRIES, SCR_BLOCK_SLOTS, SCR_TILE_COUNT };
 template <class T>
 int pct_scratch(pct_ctx* ctx, ScratchSlot slot, T** p, size_t count)
 {

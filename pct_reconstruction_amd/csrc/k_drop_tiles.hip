@@ -49,11 +49,24 @@ constexpr int kRound = 128;         // list entries cut at a time; a segment nev
 // against 83.8 us and 25.6 against 40.8 ms.  Below, a tile's own costs (its voxels read and written, its
 // descriptor) outweigh the gathers that it saves.
 constexpr double kMinSlots = 1000.0;
+// of a block: below, its kernels are as short by sorted lists.  Lists built and 20 iterations, tiles to sorted lists:
+// 128 x 128 with 0.77M slots 1.04 to 1.08, 144 x 144 with 0.88M 1.00, 160 x 160 with 0.97M 0.95.
+constexpr double kMinBlockSlots = 0.9e6;
+// of a block for every path through its busiest tile: that tile's workgroup holds up the pass, where few tiles, or few
+// crowded ones, take all the paths.  With 760 slots (64 x 64 x 12) an iteration, tiles to sorted lists, 1.24 and with the
+// lists built for 20 of them 1.23, 2860 (100 x 100 x 38) 1.39 and 1.30, 5820 to 6360 1.06 to 1.23 and 1.01 to 1.15, 7750
+// to 7990 0.99 to 1.08 and 0.94 to 1.01, 9250 to 9990 0.92 to 1.06 and 0.88 to 1.01, 13000 and more 0.90 to 0.95 and
+// 0.86 to 0.89.
+constexpr double kMinSpread = 8500.0;
+// Paths through the busiest tile (a block's mean) from which another block will have more segments there than kMaxSeg.
+// Plans with 600 and more either did not fit (616 to 1600 of them), at 2.6 ms and more for the build until that was
+// known, or gained nothing (600: 1.00, 674: 1.10, 813: 1.08); with 542, 981 segments: 0.77.
+constexpr double kMaxPaths = 600.0;
 // and of the whole plan: below, the build's fixed launches and waits cost more than the sort of so few entries
 // (head, 7M slots: list build 1.8 against 1.3 ms; cylinder-2M, 255M slots in blocks of 12800: 6.7 against 9.7 ms).
 constexpr int64_t kMinTotalSlots = 1ll << 25;
 constexpr int32_t kMaxBlock = 1 << 22;  // histories of a block (22 bits of the fill's history order)
-constexpr int64_t kSample = 1 << 16;    // paths that the rule looks at
+constexpr int64_t kSample = 1 << 14;    // paths that the rule looks at
 constexpr int64_t kSlack = 2048;       // readable elements past the lists (see k_tile_pass)
 constexpr int kMaxDup = 64;         // repeated visits of a voxel by one segment, per tile
 
@@ -122,7 +135,7 @@ __global__ void k_tile_block_caps(int64_t n_raw, int64_t BS, int64_t n,
     first[rb] = off[rb * BS];
 }
 
-// Marks the tiles of a sample of the paths: of every 8th entry of their lists, or, before the lists exist, of
+// Counts a sample of the paths through every tile, by every 8th entry of their lists, or, before the lists exist, by
 // points 8 voxels apart on their chords (the u-step is half a voxel).
 struct SampleArgs {
     int64_t n, every;
@@ -132,12 +145,17 @@ struct SampleArgs {
     const int64_t* off;
     const uint32_t *cnt, *vox;
 };
-__global__ void k_tile_sample(SampleArgs a, uint8_t* __restrict__ used)
+__global__ void k_tile_sample(SampleArgs a, uint32_t* __restrict__ count)
 {
     const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * a.every;
     if (i >= a.n) return;
+    uint32_t last = ~0u;
+    auto through = [&](uint32_t tile) {
+        if (tile != last) atomicAdd(&count[tile], 1u);
+        last = tile;
+    };
     if (!a.x0) {
-        for (uint32_t j = 0; j < a.cnt[i]; j += 8) used[tile_slot(a.vox[a.off[i] + j], a.g) >> 9] = 1;
+        for (uint32_t j = 0; j < a.cnt[i]; j += 8) through(tile_slot(a.vox[a.off[i] + j], a.g) >> 9);
         return;
     }
     const DevGeom& g = a.geom;
@@ -147,7 +165,30 @@ __global__ void k_tile_sample(SampleArgs a, uint8_t* __restrict__ used)
         const double f = (double)k / steps;
         const int x = pct_calc_voxel(g.X0, a.x0[i] + f * dx, g.VW), y = pct_calc_voxel(g.Y0, a.y0[i] + f * dy, g.VH),
                   z = pct_calc_voxel(g.Z0, a.z0[i] + f * dz, g.VT);
-        if (x < g.C && y < g.R && z < g.S) used[(((uint32_t)z >> 1) * a.g.nty + ((uint32_t)y >> 4)) * a.g.ntx + ((uint32_t)x >> 4)] = 1;
+        if (x < g.C && y < g.R && z < g.S)
+            through((((uint32_t)z >> 1) * a.g.nty + ((uint32_t)y >> 4)) * a.g.ntx + ((uint32_t)x >> 4));
+    }
+}
+
+// out[0]: the tiles with a path, out[1]: the most paths through one
+__global__ void __launch_bounds__(kBlock) k_tile_reach(uint32_t nt, const uint32_t* __restrict__ count,
+                                                       uint32_t* __restrict__ out)
+{
+    uint32_t most = 0, reached = 0;
+    for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < nt; t += gridDim.x * kBlock) {
+        const uint32_t c = count[t];
+        reached += c > 0;
+        most = c > most ? c : most;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t m = __shfl_xor(most, o, 64);
+        reached += __shfl_xor(reached, o, 64);
+        most = m > most ? m : most;
+    }
+    if ((threadIdx.x & 63) == 0 && reached) {
+        atomicAdd(out, reached);
+        atomicMax(out + 1, most);
     }
 }
 
@@ -1178,27 +1219,29 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
     PCT_TRY(pct_read(ctx, first_slot.data(), slot_dev, n_raw * sizeof(int64_t)));
     int64_t slots = 0;
     for (int64_t rb = 0; rb < n_raw; rb++) slots += cap[rb];
-    const int64_t nb_est = std::max<int64_t>(1, n / BS);
-    // The rule: list slots of a block per tile that the paths reach (see kMinSlots)
+    const double nb_est = std::max(1.0, (double)n / BS);
+    // The rule, on list slots of a block and the sampled paths through the tiles (see kMinSlots and the constants after it)
     double density = 0.0;
     if (ctx->drop_tiles != 1) {
-        uint8_t* mark = nullptr;
-        PCT_TRY(pct_scratch(ctx, SCR_TILE_MARK, &mark, g.nt));
-        PCT_CHECK_HIP(ctx, hipMemsetAsync(mark, 0, g.nt, s));
+        uint32_t* count = nullptr;  // then the reached tiles and the most paths
+        PCT_TRY(pct_scratch(ctx, SCR_TILE_COUNT, &count, (size_t)g.nt + 2));
+        PCT_CHECK_HIP(ctx, hipMemsetAsync(count, 0, ((size_t)g.nt + 2) * sizeof(uint32_t), s));
         SampleArgs a{n, (n + kSample - 1) / kSample, g, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, pct_geom(P),
                      ctx->list_off, ctx->list_cnt, ctx->list_vox};
         if (pipe) {
             a.x0 = ctx->h[0], a.y0 = ctx->h[1], a.z0 = ctx->h[2];
             a.x1 = ctx->h[3], a.y1 = ctx->h[4], a.z1 = ctx->h[5];
         }
-        hipLaunchKernelGGL(k_tile_sample, dim3(grid_for((n + a.every - 1) / a.every)), dim3(kBlock), 0, s, a, mark);
-        std::vector<uint8_t> m(g.nt);
-        PCT_TRY(pct_read(ctx, m.data(), mark, g.nt));
-        int64_t reached = 0;
-        for (uint8_t v : m) reached += v;
-        density = (double)slots / nb_est / (double)std::max<int64_t>(1, reached);
+        hipLaunchKernelGGL(k_tile_sample, dim3(grid_for((n + a.every - 1) / a.every)), dim3(kBlock), 0, s, a, count);
+        hipLaunchKernelGGL(k_tile_reach, dim3(std::min(grid_for(g.nt), 256u)), dim3(kBlock), 0, s, g.nt, count, count + g.nt);
+        uint32_t reach[2];
+        PCT_TRY(pct_read(ctx, reach, count + g.nt, sizeof(reach)));
+        const double block_slots = (double)slots / nb_est, paths = (double)reach[1] * a.every / nb_est;
+        density = block_slots / std::max(1u, reach[0]);
+        if (density < kMinSlots || block_slots < kMinBlockSlots || block_slots < kMinSpread * paths ||
+            paths >= kMaxPaths || density >= T.too_dense)
+            return PCT_OK;
     }
-    if (ctx->drop_tiles != 1 && (density < kMinSlots || density >= T.too_dense)) return PCT_OK;
 
     // groups of whole blocks
     D.blocks.clear();
