@@ -129,6 +129,14 @@ int pct_ctx_create(const pct_params* p, int device, pct_ctx** out)
         int t = std::atoi(e);
         if (t >= -1 && t <= 1) ctx->carve_tiles = t;
     }
+    if (const char* e = std::getenv("PCT_CARVE_BATCH")) {
+        long long b = std::atoll(e);
+        if (b >= 1 && b <= (4 << 20)) ctx->carve_batch = b;
+    }
+    if (const char* e = std::getenv("PCT_CARVE_BATCHES")) {
+        int b = std::atoi(e);
+        if (b >= -1) ctx->carve_batches = b;
+    }
     if (const char* e = std::getenv("PCT_CARVE_BLOCK")) {
         int t = std::atoi(e);
         if (t == 256 || t == 512) ctx->carve_block = t;
@@ -612,6 +620,9 @@ const char* pct_metrics_json(pct_ctx* ctx)
     std::snprintf(buf, sizeof(buf), ", \"drop_plan\": {\"flags\": %d, \"groups_bucketed\": %lld, \"groups_sorted\": %lld, \"tiles\": %s, \"row_lanes\": %d}",
                   ctx->plan.flags, (long long)ctx->plan.groups_bucketed, (long long)ctx->plan.groups_sorted,
                   ctx->plan.tile.ready ? "true" : "false", ctx->drop_row_lanes);
+    s += buf;
+    std::snprintf(buf, sizeof(buf), ", \"carve\": {\"by_tiles\": %lld, \"tile_batches\": %lld, \"by_walks\": %lld}",
+                  (long long)ctx->carve_by_tiles, (long long)ctx->carve_tile_batches, (long long)ctx->carve_by_walks);
     s += buf;
     double tvs_ms = 0;
     for (const TvsRecord& r : ctx->tvs_log) tvs_ms += r.ms;

@@ -260,7 +260,11 @@ struct pct_ctx {
     int carve_table = 8192;   // LDS hash slots of the fused carve (4096, 8192, 16384); 0: one walk per method (PCT_CARVE_TABLE)
     int mlp_lanes = 0;         // lanes per history of the MLP list kernels: 0 by rule, 1, 4, 16 (PCT_MLP_LANES)
     int carve_tiles = -1;      // hull carving by tiles: -1 by rule, 0 never, 1 always (PCT_CARVE_TILES)
+    int64_t carve_batch = 4 << 20;  // histories counted by tiles at a time (PCT_CARVE_BATCH)
+    int carve_batches = -1;    // batches counted by tiles, the table takes the rest; -1: all (PCT_CARVE_BATCHES)
     CarveScratch carve;
+    // the last carve: histories counted by tiles, in how many batches, and by the table or single walks
+    int64_t carve_by_tiles = 0, carve_tile_batches = 0, carve_by_walks = 0;
     int carve_line_order = 1;  // hull carving in chord-line order (both directions of a line together; PCT_CARVE_LINES)
     int endpoint_order = 1;   // MLP endpoints in sinogram-bin order (PCT_ENDPOINT_ORDER)
     int carve_block = 512;    // lanes per workgroup of the fused carve (256, 512; PCT_CARVE_BLOCK)

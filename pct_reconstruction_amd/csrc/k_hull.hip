@@ -604,7 +604,7 @@ void carve_tiles_free(CarveScratch& W)
 }
 
 // The counts by tiles, in batches of histories (in visiting order ctx->u32_d).  *done: the histories counted; fewer
-// than n, with PCT_OK, where there was no memory for the rest.
+// than n, with PCT_OK, where there was no memory for the rest or the batches are limited.
 int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gates& gt, int64_t n, int64_t* done)
 {
     hipStream_t s = ctx->stream;
@@ -613,7 +613,7 @@ int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gat
     const int64_t tiles = (int64_t)ntx * nty * ntz;
     const uint32_t n_tiles = (uint32_t)tiles;
     // 4M histories (0.9 GB on the 256 x 256 head grid), fewer where a chord may pass very many tiles
-    const int64_t kBatch = std::min<int64_t>(4 << 20, (int64_t)(1 << 28) / (2 + ntx + nty + ntz));
+    const int64_t batch = std::min<int64_t>(ctx->carve_batch, (int64_t)(1 << 28) / (2 + ntx + nty + ntz));
     int bits = 1;
     while ((1ll << bits) < tiles + 1) bits++;
     auto grow = [&](auto** p, int64_t* cap, int64_t need) -> int {
@@ -631,7 +631,8 @@ int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gat
         return (int)PCT_OK;
     };
     for (*done = 0; *done < n;) {
-        const int64_t m = std::min(kBatch, n - *done);
+        if (ctx->carve_tile_batches == ctx->carve_batches) return PCT_OK;
+        const int64_t m = std::min(batch, n - *done);
         size_t scan = 0, sort = 0;
         int rc = grow(&W.recs, &W.cap_recs, m);
         if (rc == PCT_OK) rc = grow(&W.cap, &W.cap_cap, m + 1);
@@ -677,6 +678,7 @@ int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gat
             PCT_CHECK_HIP(ctx, hipGetLastError());
         }
         *done += m;
+        ctx->carve_tile_batches++;
     }
     return PCT_OK;
 }
@@ -706,7 +708,9 @@ int pct_carve_counts(pct_ctx* ctx)
         PCT_TRY(pct_alloc(ctx, &ctx->sm_counts, NV));
         hipLaunchKernelGGL(k_init_counts, dim3(grid_for(NV)), dim3(kBlock), 0, s, g, ctx->sm_counts);
     }
+    ctx->carve_by_tiles = ctx->carve_tile_batches = ctx->carve_by_walks = 0;
     if (n > 0 && (P.sc_on || P.msc_on || P.sm_on)) {
+        ctx->carve_by_walks = n;
         if (ctx->carve_table && NV < (int64_t)kEmpty && n <= 0x7fffffff) {
             // histories in sinogram-bin order (a sort of up to 2^31 - 1); voxel numbers are 32-bit table keys
             // below kEmpty
@@ -717,6 +721,8 @@ int pct_carve_counts(pct_ctx* ctx)
                      P.msc_upper_threshold, P.sm_lower_threshold, (uint32_t)ctx->carve_spill};
             int64_t done = 0;
             if (tiles) PCT_TRY(carve_by_tiles(ctx, g, hp, gt, n, &done));
+            ctx->carve_by_tiles = done;
+            ctx->carve_by_walks = n - done;
             const int tb = ctx->carve_table, bs = ctx->carve_block;
             auto kern = tb == 4096    ? (bs == 512 ? k_carve_all<4096, 512> : k_carve_all<4096, 256>)
                         : tb == 16384 ? (bs == 512 ? k_carve_all<16384, 512> : k_carve_all<16384, 256>)
