@@ -7,7 +7,7 @@
 // traversals with 32-bit integer atomics, which are exact and order independent.  By default one walk
 // serves every method, the histories in sinogram-bin order, with the visits of a workgroup summed in
 // LDS first: in a hash table (k_carve_all; 3.4x faster than one walk per method on the head-50M workload), or, for MSC and
-// SM counts from 2^18 histories on, in the counts of an image tile that the chords pass through (k_carve_tiles).
+// SM counts of many histories on fine grids, in the counts of an image tile that the chords pass through (k_carve_tiles).
 #include <hipcub/hipcub.hpp>
 
 #include "internal.h"
@@ -592,6 +592,17 @@ namespace {
 // reconstruction: 65.3 ms by table, 66.0 by tiles).
 constexpr int64_t kCarveTilesMin = 1 << 18;
 
+// On coarse grids a workgroup's chords share their voxels, the table's counts stay in LDS and a chord has too few visits
+// to pay for its entries and their sort.  Binning and carve by table | tiles, ms, MSC and SM unless noted, with the
+// histories per voxel: 64 x 64 x 24 0.3M (3) 0.51 | 0.52, 4M (41) 1.46 | 2.03; 64 x 64 x 48 1M (5) 0.93 | 0.80, SM alone
+// 0.64 | 0.86; 96 x 96 x 64 4M (7) 2.68 | 2.70, 12M (20) 6.1 | 7.7; 128 x 128 x 24 4M (10) 2.99 | 2.89, SM alone
+// 2.37 | 2.26, 12M (31) 7.0 | 8.4; 128 x 128 x 96 12M (8) 11.4 | 9.3; 180 x 180 x 24 12M (15) 11.3 | 10.4.
+bool carve_tiles_worth(const pct_params& P, int64_t n)
+{
+    const int64_t methods = (P.msc_on != 0) + (P.sm_on != 0), sides = P.columns + P.rows;
+    return n >= kCarveTilesMin && methods * sides >= 200 && 23 * n <= sides * P.num_voxels;
+}
+
 void carve_tiles_free(CarveScratch& W)
 {
     pct_free(&W.recs);
@@ -714,8 +725,8 @@ int pct_carve_counts(pct_ctx* ctx)
         if (ctx->carve_table && NV < (int64_t)kEmpty && n <= 0x7fffffff) {
             // histories in sinogram-bin order (a sort of up to 2^31 - 1); voxel numbers are 32-bit table keys
             // below kEmpty
-            const bool worth = (P.msc_on || P.sm_on) && n >= kCarveTilesMin;
-            const bool tiles = (ctx->carve_tiles == 1 || (ctx->carve_tiles < 0 && worth)) && NV <= 0x7fffffff;
+            const bool tiles = (ctx->carve_tiles == 1 || (ctx->carve_tiles < 0 && carve_tiles_worth(P, n))) &&
+                               NV <= 0x7fffffff;
             PCT_TRY(ctx->carve_line_order && !tiles ? pct_line_order(ctx, n) : pct_bin_order(ctx, n));
             Gates gt{P.sc_on, P.msc_on, P.sm_on, P.sc_lower_threshold, P.sc_upper_threshold, P.msc_lower_threshold,
                      P.msc_upper_threshold, P.sm_lower_threshold, (uint32_t)ctx->carve_spill};
