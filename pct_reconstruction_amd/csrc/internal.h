@@ -208,12 +208,14 @@ struct alignas(32) CarveRec {  // one history in visiting order
     uint32_t inc;  // MSC | SM << 15 | SC << 30
     float pad;
 };
-struct CarveScratch {  // kept until the reconstruction volume is complete; bounded by a batch of histories
+struct CarveScratch {  // bounded by a batch of histories; stays for the next run up to kCarveKeep
     CarveRec* recs = nullptr;
     uint32_t *cap = nullptr, *off = nullptr, *keys = nullptr, *tiles = nullptr;
     uint64_t* vals = nullptr;
     int64_t cap_recs = 0, cap_cap = 0, cap_off = 0, cap_keys = 0, cap_tiles = 0, cap_vals = 0;
+    bool busy = false;
 };
+constexpr int64_t kCarveKeep = 1ll << 30;  // bytes
 
 struct pct_ctx {
     pct_params P;
@@ -402,6 +404,7 @@ struct pct_tmp {
 
 DevGeom pct_geom(const pct_params& P);
 void pct_carve_free(pct_ctx* ctx);              // the carve's scratch
+int64_t pct_carve_bytes(const pct_ctx* ctx);    // its size
 // The first `bytes` at src on the device, once the stream is done: through pinned memory where they are few (a copy to
 // pageable memory stages and waits for itself, 10 us more).
 constexpr size_t kReadBytes = 4096;

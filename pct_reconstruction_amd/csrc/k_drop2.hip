@@ -869,13 +869,23 @@ static void free_lists(DropPlan* D)
     D->cap_entries = D->cap_off = D->cap_r = D->cap_perm = D->cap_group_e = D->cap_group_h = D->cap_group_b = 0;
 }
 
+// the arrays of the plan that is not in use; true if there were any
+static bool free_idle(DropPlan* D)
+{
+    const bool any = D->idle != DropPlan::IDLE_NONE;
+    if (D->idle == DropPlan::IDLE_LISTS) free_lists(D);
+    if (D->idle == DropPlan::IDLE_TILES) pct_tile_plan_free(&D->tile);
+    D->idle = DropPlan::IDLE_NONE;
+    return any;
+}
+
 bool pct_give_back(pct_ctx* ctx)
 {
-    DropPlan& D = ctx->plan;
-    const bool any = D.idle != DropPlan::IDLE_NONE;
-    if (D.idle == DropPlan::IDLE_LISTS) free_lists(&D);
-    if (D.idle == DropPlan::IDLE_TILES) pct_tile_plan_free(&D.tile);
-    D.idle = DropPlan::IDLE_NONE;
+    bool any = free_idle(&ctx->plan);
+    if (!ctx->carve.busy && pct_carve_bytes(ctx) > 0) {
+        pct_carve_free(ctx);
+        any = true;
+    }
     return any;
 }
 
@@ -970,14 +980,14 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
             // the sorted lists are those of an earlier plan with other flags, or of a sparser segment: every iteration
             // comes back to that one (large grid, two segments of 473K histories by tiles and one of 40K by lists: an
             // iteration 15.2 ms, 24.2 with each plan freed for the other)
-            if (!ctx->seg_inside) pct_give_back(ctx);
+            if (!ctx->seg_inside) free_idle(&D);
             return PCT_OK;
         }
         if (built) mlp = nullptr;  // the lists exist now
     }
     D.tile.ready = false;
     D.idle = DropPlan::IDLE_TILES;
-    if (!ctx->seg_inside) pct_give_back(ctx);
+    if (!ctx->seg_inside) free_idle(&D);
     const bool pipe = mlp != nullptr;  // the lists are built group by group below
     const int64_t BS = P.drop_block_size;
     D.blocks.clear();

@@ -698,6 +698,12 @@ int carve_by_tiles(pct_ctx* ctx, const DevGeom& g, const HistPtrs& hp, const Gat
 
 void pct_carve_free(pct_ctx* ctx) { carve_tiles_free(ctx->carve); }
 
+int64_t pct_carve_bytes(const pct_ctx* ctx)
+{
+    const CarveScratch& W = ctx->carve;
+    return W.cap_recs * (int64_t)sizeof(CarveRec) + (W.cap_cap + W.cap_off + W.cap_keys + W.cap_tiles) * 4 + W.cap_vals * 8;
+}
+
 // hull_initializations (DS.cu:6636) + the carving counts of hull_detection (:6607)
 int pct_carve_counts(pct_ctx* ctx)
 {
@@ -731,7 +737,12 @@ int pct_carve_counts(pct_ctx* ctx)
             Gates gt{P.sc_on, P.msc_on, P.sm_on, P.sc_lower_threshold, P.sc_upper_threshold, P.msc_lower_threshold,
                      P.msc_upper_threshold, P.sm_lower_threshold, (uint32_t)ctx->carve_spill};
             int64_t done = 0;
-            if (tiles) PCT_TRY(carve_by_tiles(ctx, g, hp, gt, n, &done));
+            if (tiles) {
+                ctx->carve.busy = true;
+                const int rc = carve_by_tiles(ctx, g, hp, gt, n, &done);
+                ctx->carve.busy = false;
+                PCT_TRY(rc);
+            }
             ctx->carve_by_tiles = done;
             ctx->carve_by_walks = n - done;
             const int tb = ctx->carve_table, bs = ctx->carve_block;
