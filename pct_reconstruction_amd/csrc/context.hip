@@ -160,6 +160,13 @@ int pct_ctx_create(const pct_params* p, int device, pct_ctx** out)
         int l = std::atoi(e);
         if (l == 1 || l == 4 || l == 16) ctx->mlp_lanes = l;
     }
+    if (const char* e = std::getenv("PCT_FAIL_ALLOCATIONS")) {
+        long long first = 0, count = 0;
+        if (std::sscanf(e, "%lld,%lld", &first, &count) == 2) {
+            ctx->fail_first = first;
+            ctx->fail_count = count;
+        }
+    }
     if (const char* e = std::getenv("PCT_DROP_GROUP_ENTRIES")) {
         long long g = std::atoll(e);
         if (g >= 1 && g <= (1ll << 30)) ctx->drop_group_entries = g;
@@ -678,6 +685,15 @@ int pct_drop_iteration_device(int64_t n, const int64_t* offsets, const uint32_t*
 }
 
 }  // extern "C"
+
+hipError_t pct_malloc(pct_ctx* ctx, void** p, size_t bytes)
+{
+    const int64_t k = ++ctx->allocations - ctx->fail_first;
+    if (k >= 0 && k < ctx->fail_count) return hipErrorOutOfMemory;
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
 
 int pct_read(pct_ctx* ctx, void* dst, const void* src, size_t bytes)
 {

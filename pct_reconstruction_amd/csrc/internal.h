@@ -50,6 +50,7 @@ struct DevTables {
     double* step_terms = nullptr;  // [k][8]: u1_12, u1_23, p34(u1), S1I0, S1I1, S1I2, unused, unused
     int n_steps = 0;               // rows of step_terms
     int64_t n_trig = 0, n_coeff = 0, n_poly = 0;
+    bool ready = false;  // all of them are there
 };
 
 // Per history, in visiting order: what the row kernel needs before its list (one 24-byte load).
@@ -254,6 +255,7 @@ struct pct_ctx {
     void* cub_tmp = nullptr;
     uint8_t* scratch[6] = {};      // by ScratchSlot
     int64_t allocations = 0;       // device allocations made for the context (metrics)
+    int64_t fail_first = 0, fail_count = 0;  // those that report no memory, for tests (PCT_FAIL_ALLOCATIONS=first,count)
     void* read_h = nullptr;        // pinned, kReadBytes: where small results land (pct_read)
     double* angle_cs = nullptr;    // cos and sin of the angle bins, as the binning and as the FBP form them
     size_t cub_tmp_bytes = 0;
@@ -347,6 +349,8 @@ struct pct_ctx {
 // allocation helpers
 // Frees what the context keeps only to use it again (no memory); true if there was any.
 bool pct_give_back(pct_ctx* ctx);
+// hipMalloc, counted; leaves no error behind.
+hipError_t pct_malloc(pct_ctx* ctx, void** p, size_t bytes);
 // A buffer that is there already and holds `count` elements, with at most a quarter and 64 KB to spare, stays: a
 // context that runs its stages again asks for the same sizes, and a free and an allocation took 10 to 60 us each
 // time, 33 times in a reconstruction.
@@ -364,12 +368,8 @@ int pct_alloc(pct_ctx* ctx, T** p, size_t count)
         (void)hipFree(*p);
         *p = nullptr;
     }
-    hipError_t e = hipMalloc((void**)p, count * sizeof(T));
-    ctx->allocations++;
-    if (e != hipSuccess && pct_give_back(ctx)) {
-        (void)hipGetLastError();
-        e = hipMalloc((void**)p, count * sizeof(T));
-    }
+    hipError_t e = pct_malloc(ctx, (void**)p, count * sizeof(T));
+    if (e != hipSuccess && pct_give_back(ctx)) e = pct_malloc(ctx, (void**)p, count * sizeof(T));
     if (e != hipSuccess) {
         ctx->err = std::string("hipMalloc(") + std::to_string(count * sizeof(T)) + " B): " + hipGetErrorString(e);
         *p = nullptr;

@@ -809,10 +809,7 @@ int build_slices(pct_ctx* ctx, DropPlan& D)
         hipLaunchKernelGGL(k_slice_width, dim3(grid), dim3(kWave), 0, s, NS, chunk, nb, D.slice_blocks, D.t_off, w);
     size_t tb = 0;
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, tb, w, D.sell_off, (int)(NS + 1), s));
-    if (tb > ctx->cub_tmp_bytes) {
-        PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, tb));
-        ctx->cub_tmp_bytes = tb;
-    }
+    PCT_TRY(pct_grow_cub(ctx, tb));
     tb = ctx->cub_tmp_bytes;
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, tb, w, D.sell_off, (int)(NS + 1), s));
     uint64_t total = 0;
@@ -1090,6 +1087,7 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
         D.cap_perm = n + 1;
     }
     if (D.cap_group_e < max_ge + 1 || !D.keys) {
+        D.cap_group_e = 0;
         PCT_TRY(pct_alloc(ctx, &D.keys, max_ge + 1));
         PCT_TRY(pct_alloc(ctx, &D.keys_sorted, max_ge + 1));
         PCT_TRY(pct_alloc(ctx, &D.vals, max_ge + 1));
@@ -1097,6 +1095,7 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
         D.cap_group_e = max_ge + 1;
     }
     if (D.cap_group_h < max_gh + 1 || !D.hkey) {
+        D.cap_group_h = 0;
         PCT_TRY(pct_alloc(ctx, &D.hkey, max_gh + 1));
         PCT_TRY(pct_alloc(ctx, &D.hkey_sorted, max_gh + 1));
         PCT_TRY(pct_alloc(ctx, &D.hidx, max_gh + 1));
@@ -1144,6 +1143,7 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
             return PCT_E_LIMIT;
         }
         if (D.cap_bk < nbk || !D.bk_cnt) {
+            D.cap_bk = 0;
             PCT_TRY(pct_alloc(ctx, &D.bk_cnt, nbk));
             PCT_TRY(pct_alloc(ctx, &D.bk_off, nbk));
             PCT_TRY(pct_alloc(ctx, &D.bk_cur, nbk));
@@ -1176,10 +1176,7 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
         need = std::max(need, t);
         PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, t, D.runs, D.t_off, E1, s));
         need = std::max(need, t);
-        if (need > ctx->cub_tmp_bytes) {
-            PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, need));
-            ctx->cub_tmp_bytes = need;
-        }
+        PCT_TRY(pct_grow_cub(ctx, need));
     }
     std::vector<std::vector<int32_t>> run_start_h(ng);
     std::vector<uint32_t> n_runs_h(ng, 0);
@@ -1569,10 +1566,7 @@ int pct_stage_residual(pct_ctx* ctx, double* norm)
         PCT_CHECK_HIP(ctx, hipGetLastError());
         size_t need = 0;
         PCT_CHECK_HIP(ctx, hipcub::DeviceReduce::Sum(nullptr, need, ctx->res_r2, out, n, s));
-        if (need > ctx->cub_tmp_bytes) {
-            PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, need));
-            ctx->cub_tmp_bytes = need;
-        }
+        PCT_TRY(pct_grow_cub(ctx, need));
         need = ctx->cub_tmp_bytes;
         PCT_CHECK_HIP(ctx, hipcub::DeviceReduce::Sum(ctx->cub_tmp, need, ctx->res_r2, out, n, s));
     }

@@ -733,7 +733,7 @@ int pct_stage_endpoints(pct_ctx* ctx)
 
 static int upload_tables(pct_ctx* ctx)
 {
-    if (ctx->T.sin_t) return PCT_OK;
+    if (ctx->T.ready) return PCT_OK;
     const pct_params& P = ctx->P;
     hipStream_t s = ctx->stream;
     HostTables ht;
@@ -764,6 +764,7 @@ static int upload_tables(pct_ctx* ctx)
     PCT_CHECK_HIP(ctx, up(T.p312, ht.p312));
     PCT_CHECK_HIP(ctx, up(T.step_terms, terms));
     PCT_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    T.ready = true;
     return PCT_OK;
 }
 
@@ -780,6 +781,9 @@ int pct_stage_build_lists(pct_ctx* ctx)
         ctx->stage = ST_LISTS;
         return PCT_OK;
     }
+    // the lists and the plan over them are replaced: until that has succeeded there are none
+    ctx->plan.ready = false;
+    if (!ctx->seg_inside) ctx->stage = ST_ENDPOINTS;
     MlpArgs a;
     a.g = pct_geom(P);
     a.trig_min = P.trig_table_min;
@@ -796,6 +800,7 @@ int pct_stage_build_lists(pct_ctx* ctx)
     H10 hp;
     for (int k = 0; k < 10; k++) hp.h[k] = ctx->h[k];
     if (n > ctx->list_hist_cap || !ctx->list_off) {  // buffers persist across rebuilds
+        ctx->list_hist_cap = 0;
         PCT_TRY(pct_alloc(ctx, &ctx->list_off, n + 1));
         PCT_TRY(pct_alloc(ctx, &ctx->list_cnt, n));
         PCT_TRY(pct_alloc(ctx, &ctx->chord, n));
@@ -816,14 +821,12 @@ int pct_stage_build_lists(pct_ctx* ctx)
                            ctx->T.cos_t, capv);
     size_t need = 0;
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, need, capv, ctx->list_off, n + 1, s));
-    if (need > ctx->cub_tmp_bytes) {
-        PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, need));
-        ctx->cub_tmp_bytes = need;
-    }
+    PCT_TRY(pct_grow_cub(ctx, need));
     PCT_CHECK_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->cub_tmp, need, capv, ctx->list_off, n + 1, s));
     int64_t total = 0;
     PCT_TRY(pct_read(ctx, &total, ctx->list_off + n, sizeof(int64_t)));
     if (total > ctx->list_cap) {
+        ctx->list_cap = 0;
         PCT_TRY(pct_alloc(ctx, &ctx->list_vox, total));
         ctx->list_cap = total;
     }

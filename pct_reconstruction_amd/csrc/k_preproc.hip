@@ -501,10 +501,7 @@ int pct_line_order(pct_ctx* ctx, int64_t n)
         size_t need = 0;
         PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, need, ctx->u32_a, ctx->u32_b, ctx->u32_c,
                                                               ctx->u32_d, (int)n, 0, end_bit, s));
-        if (need > ctx->cub_tmp_bytes) {
-            PCT_TRY(pct_alloc(ctx, (uint8_t**)&ctx->cub_tmp, need));
-            ctx->cub_tmp_bytes = need;
-        }
+        PCT_TRY(pct_grow_cub(ctx, need));
         PCT_CHECK_HIP(ctx, hipcub::DeviceRadixSort::SortPairs(ctx->cub_tmp, need, ctx->u32_a, ctx->u32_b, ctx->u32_c,
                                                               ctx->u32_d, (int)n, 0, end_bit, s));
         PCT_CHECK_HIP(ctx, hipGetLastError());
@@ -515,6 +512,7 @@ int pct_line_order(pct_ctx* ctx, int64_t n)
 int pct_ensure_hist_capacity(pct_ctx* ctx, int64_t n)
 {
     if (n <= ctx->cap_hist) return PCT_OK;
+    ctx->cap_hist = 0;  // until they all are there
     for (int k = 0; k < 10; k++) {
         PCT_TRY(pct_alloc(ctx, &ctx->h[k], n));
         PCT_TRY(pct_alloc(ctx, &ctx->h_tmp[k], n));
@@ -571,6 +569,7 @@ int pct_stage_intersect_bin_carve(pct_ctx* ctx)
     const pct_params& P = ctx->P;
     hipStream_t s = ctx->stream;
     const int64_t n = ctx->n_loaded;
+    ctx->stage = ST_LOADED;  // the histories of an earlier run are overwritten
     PCT_TRY(pct_ensure_hist_capacity(ctx, n));
     ctx->bin_perm_n = -1;
     unsigned g = grid_for(n);

@@ -311,6 +311,7 @@ extern "C" int pct_import_preprocessed(pct_ctx* ctx, const char* dir)
     // device state: per-history arrays, lists, images
     PCT_TRY(pct_ensure_hist_capacity(ctx, n));
     if (n > ctx->list_hist_cap || !ctx->list_off) {
+        ctx->list_hist_cap = 0;
         PCT_TRY(pct_alloc(ctx, &ctx->list_off, n + 1));
         PCT_TRY(pct_alloc(ctx, &ctx->list_cnt, n));
         PCT_TRY(pct_alloc(ctx, &ctx->chord, n));
@@ -318,6 +319,7 @@ extern "C" int pct_import_preprocessed(pct_ctx* ctx, const char* dir)
         ctx->list_hist_cap = n;
     }
     if (total > ctx->list_cap) {
+        ctx->list_cap = 0;
         PCT_TRY(pct_alloc(ctx, &ctx->list_vox, total));
         ctx->list_cap = total;
     }
