@@ -309,6 +309,9 @@ extern "C" int pct_import_preprocessed(pct_ctx* ctx, const char* dir)
     }
 
     // device state: per-history arrays, lists, images
+    // an earlier run's histories and lists are overwritten: until all of these are there, only loaded ones can be used
+    ctx->stage = ctx->n_loaded > 0 ? ST_LOADED : ST_EMPTY;
+    ctx->plan.ready = false;
     PCT_TRY(pct_ensure_hist_capacity(ctx, n));
     if (n > ctx->list_hist_cap || !ctx->list_off) {
         ctx->list_hist_cap = 0;
