@@ -972,7 +972,13 @@ int pct_drop_prepare(pct_ctx* ctx, const MlpLaunch* mlp)
         D.ready = false;
         D.idle = DropPlan::IDLE_LISTS;
         bool done = false, built = false;
-        PCT_TRY(pct_tiles_prepare(ctx, mlp, &done, &built));
+        const int rc = pct_tiles_prepare(ctx, mlp, &done, &built);
+        if (rc == PCT_E_NOMEM) {  // lists that change the tile at every step take more than sorted ones
+            pct_tile_plan_free(&D.tile);
+            ctx->err.clear();
+        } else if (rc != PCT_OK) {
+            return rc;
+        }
         if (done) {
             // the sorted lists are those of an earlier plan with other flags, or of a sparser segment: every iteration
             // comes back to that one (large grid, two segments of 473K histories by tiles and one of 40K by lists: an
