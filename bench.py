@@ -661,7 +661,13 @@ def main() -> int:
                                           "drop_block (k_drop_rows + k_drop_cols per DROP block)"),
                 "achieved": block_bytes / (block_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": block_bytes / (block_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": traffic,
-                "traffic_source": traffic_src, "bytes_per_launch": block_bytes, "avg_launch_ms": block_ms}
+                "traffic_source": traffic_src, "bytes_per_launch": block_bytes, "avg_launch_ms": block_ms,
+                # achieved and frac price the reference's bytes, of which tiles move about two thirds; what the block
+                # moves, and what holds it up, beside them
+                "basis": "algorithmic bytes of the reference's DROP: 18 B per list entry + 12 B per history",
+                "traffic_GBs": None if traffic is None else traffic / (block_ms * 1e-3) / 1e9,
+                "traffic_frac": None if traffic is None else traffic / (block_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+                "limit": "latency" if tiles else "gather rate"}
     # whole-step algorithmic HBM rate: list writes (4 B per entry + 64 B per history) and the DROP blocks
     step_bytes = iters * (block_bytes * nb) + (iters if segs else 1) * mlp_bytes
     hbm_step = {"GBs": step_bytes / (ms_per_step * 1e-3) / 1e9, "bytes_per_step": step_bytes}

@@ -511,7 +511,7 @@ __global__ void k_mlp_capacity_std(int64_t n, StdArgs a, H10 hp, int64_t* cap)
     cap[i] = 1 + steps;
 }
 
-// One history per lane, grid-stride.  FP64 throughout, with the reference's float powf roundings.
+// G lanes per history, grid-stride.  FP64 throughout, with the reference's float powf roundings.
 template <int G>
 __global__ void __launch_bounds__(kBlock) k_mlp_lists_std(int64_t n, StdArgs a, H10 hp,
                                                           const uint32_t* __restrict__ first,

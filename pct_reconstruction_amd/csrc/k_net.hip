@@ -719,9 +719,9 @@ int launch_conv_as(pct_net* net, const ConvIn& in, int level, const ConvShape& s
 
 // The tile's rule.  More rows per wave use a weight fragment more often, and fewer waves along the channels an input
 // fragment; both need rows, so fewer workgroups and a larger halo.  In order of rows per wave, and with the channels
-// of 32 and 64 first on fewer waves, the first shape is taken that leaves three workgroups room on a compute unit
-// (54 KB; 64 with the granularity of the shapes) and has 384 of them; a halo of 192 channels needs more than that
-// at any useful size and may take 160 KB.  Measured (us, taken | next): on 256 x 256 x 96, 48 -> 16 channels 8 rows in
+// of 32 and 64 first on fewer waves, the first shape is taken that needs at most 64 KB of LDS, so that two or three
+// workgroups share a compute unit, and has 384 workgroups; a halo of 192 channels needs more than that at any useful
+// size and may take 160 KB.  Measured (us, taken | next): on 256 x 256 x 96, 48 -> 16 channels 8 rows in
 // 47 KB 698 | 16 rows in 71 KB 738; 96 -> 32 at half size 4 rows in 59 KB 293 | 8 in 89 KB 380; 192 -> 64 at a quarter
 // 4 rows in 115 KB 160 | 1 in 65 KB 205; 32 -> 64 there 8 rows, 768 workgroups 18.0 | 4 rows 19.9; on 128 x 128 x 32,
 // 16 -> 32 at half size 8 rows, 512 workgroups 7.7 | 16 rows, 256 workgroups 9.5.
