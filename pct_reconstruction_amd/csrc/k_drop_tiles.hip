@@ -432,7 +432,7 @@ __global__ void __launch_bounds__(kBlock) k_tile_fill(FillArgs a, TileRun* __res
                                                       unsigned long long* __restrict__ cursor,
                                                       uint32_t* __restrict__ limits, BlockTotals* __restrict__ totals)
 {
-    extern __shared__ uint32_t bits[];  // [segment / 32][voxel]
+    extern __shared__ __align__(16) uint32_t bits[];  // [segment / 32][voxel]; `hist` is read 16 bytes at a time
     __shared__ uint32_t bins[128], len_bins[kRound + 1], part[4], heads[8], row_heads[16], n_dup;
     __shared__ uint32_t dup[kMaxDup];
     __shared__ uint16_t slot_at[kTileVox], cnt_at[kTileVox];
