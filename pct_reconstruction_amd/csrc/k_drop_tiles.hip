@@ -49,18 +49,20 @@ constexpr int kRound = 128;         // list entries cut at a time; a segment nev
 // against 83.8 us and 25.6 against 40.8 ms.  Below, a tile's own costs (its voxels read and written, its
 // descriptor) outweigh the gathers that it saves.
 constexpr double kMinSlots = 1000.0;
-// of a block: below, its kernels are as short by sorted lists.  Lists built and 20 iterations, tiles to sorted lists:
-// 128 x 128 with 0.77M slots 1.04 to 1.08, 144 x 144 with 0.88M 1.00, 160 x 160 with 0.97M 0.95.
-constexpr double kMinBlockSlots = 0.9e6;
-// of a block for every path through its busiest tile: that tile's workgroup holds up the pass, where few tiles, or few
-// crowded ones, take all the paths.  With 760 slots (64 x 64 x 12) an iteration, tiles to sorted lists, 1.24 and with the
-// lists built for 20 of them 1.23, 2860 (100 x 100 x 38) 1.39 and 1.30, 5820 to 6360 1.06 to 1.23 and 1.01 to 1.15, 7750
-// to 7990 0.99 to 1.08 and 0.94 to 1.01, 9250 to 9990 0.92 to 1.06 and 0.88 to 1.01, 13000 and more 0.90 to 0.95 and
-// 0.86 to 0.89.
-constexpr double kMinSpread = 8500.0;
-// Paths through the busiest tile (a block's mean) from which another block will have more segments there than kMaxSeg.
-// Plans with 600 and more either did not fit (616 to 1600 of them), at 2.6 ms and more for the build until that was
-// known, or gained nothing (600: 1.00, 674: 1.10, 813: 1.08); with 542, 981 segments: 0.77.
+// and in blocks of few slots, whose kernels are as short by sorted lists: 128 x 128 with 0.77M slots and 1000 to 2000 in a
+// tile, lists built and 20 iterations, 1.04 to 1.08 of the sorted lists' time, 183 x 124 with 0.47M and 1440 1.02, but
+// 201 x 112 with 0.80M and 2900 0.98, 110 x 215 with 0.61M and 2400 0.96.
+constexpr double kMinSlotsSmall = 1500.0, kSmallBlock = 0.8e6;
+// Paths through the busiest tile (a block's mean): its workgroup holds up the pass where few tiles take all the paths.
+// With so many in it, a block must have kMinSpread slots for each of them.  The whole of a reconstruction, or of list
+// build and iterations, or of iterations alone, tiles to sorted lists, by that ratio: 2860 (535 paths) 1.30, 4100 (541)
+// 1.04, 4260 (340) 1.14, 5050 (387) 1.09, 5820 to 6540 (410 to 506) 1.07 to 1.15, 6930 to 8430 (280 to 410) 0.91 to
+// 0.98, 8600 to 9800 0.89 to 0.96, above 12000 at most 0.96.  With fewer paths in it: 3190 to 6410 (147 to 304) 0.96 to
+// 1.03.
+constexpr double kManyPaths = 310.0, kMinSpread = 6800.0;
+// Such paths from which another block will have more segments there than kMaxSeg.  Plans with 600 and more either did not
+// fit (614 to 2060 of them), at 2.6 ms and more for the build until that was known, or gained nothing (600: 1.00, 639:
+// 0.98, 674: 1.10, 740: 1.05, 813: 1.08); with 542, 981 segments: 0.77, with 574: 0.85.
 constexpr double kMaxPaths = 600.0;
 // and of the whole plan: below, the build's fixed launches and waits cost more than the sort of so few entries
 // (head, 7M slots: list build 1.8 against 1.3 ms; cylinder-2M, 255M slots in blocks of 12800: 6.7 against 9.7 ms).
@@ -136,7 +138,8 @@ __global__ void k_tile_block_caps(int64_t n_raw, int64_t BS, int64_t n,
 }
 
 // Counts a sample of the paths through every tile, by every 8th entry of their lists, or, before the lists exist, by
-// points 8 voxels apart on their chords (the u-step is half a voxel).
+// points 8 voxels apart on their chords (the u-step is half a voxel).  Few tiles are counted in LDS first (300 tiles on
+// 219 x 153 x 8: 98 us with every count in memory, now 12).
 struct SampleArgs {
     int64_t n, every;
     TileGeom g;
@@ -145,15 +148,10 @@ struct SampleArgs {
     const int64_t* off;
     const uint32_t *cnt, *vox;
 };
-__global__ void k_tile_sample(SampleArgs a, uint32_t* __restrict__ count)
+constexpr uint32_t kSampleTiles = 8192;  // counted in LDS
+template <class Through>
+__device__ __forceinline__ void sample_path(const SampleArgs& a, int64_t i, Through through)
 {
-    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * a.every;
-    if (i >= a.n) return;
-    uint32_t last = ~0u;
-    auto through = [&](uint32_t tile) {
-        if (tile != last) atomicAdd(&count[tile], 1u);
-        last = tile;
-    };
     if (!a.x0) {
         for (uint32_t j = 0; j < a.cnt[i]; j += 8) through(tile_slot(a.vox[a.off[i] + j], a.g) >> 9);
         return;
@@ -167,6 +165,30 @@ __global__ void k_tile_sample(SampleArgs a, uint32_t* __restrict__ count)
                   z = pct_calc_voxel(g.Z0, a.z0[i] + f * dz, g.VT);
         if (x < g.C && y < g.R && z < g.S)
             through((((uint32_t)z >> 1) * a.g.nty + ((uint32_t)y >> 4)) * a.g.ntx + ((uint32_t)x >> 4));
+    }
+}
+template <bool LDS>
+__global__ void __launch_bounds__(kBlock) k_tile_sample(SampleArgs a, uint32_t* __restrict__ count)
+{
+    extern __shared__ uint32_t local[];  // LDS: a.g.nt counts
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * a.every;
+    if (LDS) {
+        for (uint32_t t = threadIdx.x; t < a.g.nt; t += kBlock) local[t] = 0u;
+        __syncthreads();
+    }
+    uint32_t last = ~0u;
+    if (i < a.n)
+        sample_path(a, i, [&](uint32_t tile) {
+            if (tile != last) {
+                if (LDS) atomicAdd(&local[tile], 1u);
+                else atomicAdd(&count[tile], 1u);
+            }
+            last = tile;
+        });
+    if (LDS) {
+        __syncthreads();
+        for (uint32_t t = threadIdx.x; t < a.g.nt; t += kBlock)
+            if (local[t]) atomicAdd(&count[t], local[t]);
     }
 }
 
@@ -1199,6 +1221,34 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
     const int64_t max_blocks = 1ll << (32 - std::max(tile_bits, bin_bits));
     const int64_t n_raw = (n + BS - 1) / BS;
 
+    const double nb_est = std::max(1.0, (double)n / BS);
+    // The rule, on list slots of a block and the sampled paths through the tiles (see kMinSlots and the constants after it)
+    double density = 0.0;
+    if (ctx->drop_tiles != 1) {
+        uint32_t* count = nullptr;  // then the reached tiles and the most paths
+        PCT_TRY(pct_scratch(ctx, SCR_TILE_COUNT, &count, (size_t)g.nt + 2));
+        PCT_CHECK_HIP(ctx, hipMemsetAsync(count, 0, ((size_t)g.nt + 2) * sizeof(uint32_t), s));
+        SampleArgs a{n, (n + kSample - 1) / kSample, g, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, pct_geom(P),
+                     ctx->list_off, ctx->list_cnt, ctx->list_vox};
+        if (pipe) {
+            a.x0 = ctx->h[0], a.y0 = ctx->h[1], a.z0 = ctx->h[2];
+            a.x1 = ctx->h[3], a.y1 = ctx->h[4], a.z1 = ctx->h[5];
+        }
+        const dim3 sg(grid_for((n + a.every - 1) / a.every));
+        if (g.nt <= kSampleTiles)
+            hipLaunchKernelGGL(k_tile_sample<true>, sg, dim3(kBlock), g.nt * sizeof(uint32_t), s, a, count);
+        else
+            hipLaunchKernelGGL(k_tile_sample<false>, sg, dim3(kBlock), 0, s, a, count);
+        hipLaunchKernelGGL(k_tile_reach, dim3(std::min(grid_for(g.nt), 256u)), dim3(kBlock), 0, s, g.nt, count, count + g.nt);
+        uint32_t reach[2];
+        PCT_TRY(pct_read(ctx, reach, count + g.nt, sizeof(reach)));
+        const double block_slots = (double)ctx->list_slots / nb_est, paths = (double)reach[1] * a.every / nb_est;
+        density = block_slots / std::max(1u, reach[0]);
+        if (density < (block_slots < kSmallBlock ? kMinSlotsSmall : kMinSlots) ||
+            (paths >= kManyPaths && block_slots < kMinSpread * paths) || paths >= kMaxPaths || density >= T.too_dense)
+            return PCT_OK;
+    }
+
     // processed histories per raw block (DS.cu:9558 floors them) and their list capacities
     std::vector<int32_t> proc(n_raw), block_of(n_raw, -1);
     for (int64_t rb = 0; rb < n_raw; rb++) {
@@ -1217,31 +1267,6 @@ int pct_tiles_prepare(pct_ctx* ctx, const MlpLaunch* mlp, bool* done, bool* list
                        ctx->list_off, cap_dev, slot_dev);
     PCT_CHECK_HIP(ctx, hipMemcpyAsync(cap.data(), cap_dev, n_raw * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     PCT_TRY(pct_read(ctx, first_slot.data(), slot_dev, n_raw * sizeof(int64_t)));
-    int64_t slots = 0;
-    for (int64_t rb = 0; rb < n_raw; rb++) slots += cap[rb];
-    const double nb_est = std::max(1.0, (double)n / BS);
-    // The rule, on list slots of a block and the sampled paths through the tiles (see kMinSlots and the constants after it)
-    double density = 0.0;
-    if (ctx->drop_tiles != 1) {
-        uint32_t* count = nullptr;  // then the reached tiles and the most paths
-        PCT_TRY(pct_scratch(ctx, SCR_TILE_COUNT, &count, (size_t)g.nt + 2));
-        PCT_CHECK_HIP(ctx, hipMemsetAsync(count, 0, ((size_t)g.nt + 2) * sizeof(uint32_t), s));
-        SampleArgs a{n, (n + kSample - 1) / kSample, g, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, pct_geom(P),
-                     ctx->list_off, ctx->list_cnt, ctx->list_vox};
-        if (pipe) {
-            a.x0 = ctx->h[0], a.y0 = ctx->h[1], a.z0 = ctx->h[2];
-            a.x1 = ctx->h[3], a.y1 = ctx->h[4], a.z1 = ctx->h[5];
-        }
-        hipLaunchKernelGGL(k_tile_sample, dim3(grid_for((n + a.every - 1) / a.every)), dim3(kBlock), 0, s, a, count);
-        hipLaunchKernelGGL(k_tile_reach, dim3(std::min(grid_for(g.nt), 256u)), dim3(kBlock), 0, s, g.nt, count, count + g.nt);
-        uint32_t reach[2];
-        PCT_TRY(pct_read(ctx, reach, count + g.nt, sizeof(reach)));
-        const double block_slots = (double)slots / nb_est, paths = (double)reach[1] * a.every / nb_est;
-        density = block_slots / std::max(1u, reach[0]);
-        if (density < kMinSlots || block_slots < kMinBlockSlots || block_slots < kMinSpread * paths ||
-            paths >= kMaxPaths || density >= T.too_dense)
-            return PCT_OK;
-    }
 
     // groups of whole blocks
     D.blocks.clear();
